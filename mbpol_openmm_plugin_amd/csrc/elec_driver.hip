@@ -110,8 +110,8 @@ struct Elec {
     } binq;  // sites with a charge, by grid brick
     DevBuf g0tab, sptab;  // per-site spline table
     DevBuf rowcount, rowstart, rowfill, esite, ecoef;  // dipole-spreading table in grid-point order
-    // grid transforms: the LDS transforms of kernels_fft.hip when every axis
-    // factors into radices 2..13, else hipFFT
+    // grid transforms: the library's own passes (kernels_fft.hip, kernels_dft.hip) when every
+    // axis has a form there (fft_plan), else hipFFT
     PmeFft fft{};
     DevBuf tw[3];
     bool lds_fft = false;
@@ -201,7 +201,7 @@ static int up(hipStream_t stream, DevBuf& b, const std::vector<T>& v) {
     return MBPOL_OK;
 }
 
-// factor n into the radices of the LDS transforms; false if some factor is not one of them
+// factor n into the radices of the mixed-radix transforms; false if some factor is not one of them
 static bool fft_factor(int n, FftAxis& a) {
     a.n = n;
     a.nfac = 0;
@@ -211,7 +211,10 @@ static bool fft_factor(int n, FftAxis& a) {
             a.fac[a.nfac++] = p;
             r /= p;
         }
-    if (r != 1 || n > kFftMaxLength) return false;
+    if (r != 1 || n > kFftMaxLength) {
+        a.nfac = 0;  // no mixed-radix form
+        return false;
+    }
     int ns = 1, maxnb = 1;
     for (int s = 0; s < a.nfac; ++s) {
         a.ns[s] = ns;
@@ -225,6 +228,38 @@ static bool fft_factor(int n, FftAxis& a) {
     while ((1 << a.lgP) < maxnb && a.lgP < 7) ++a.lgP;
     a.inplace = (1 << a.lgP) >= maxnb;
     return true;
+}
+
+// Transforms of one axis (d = 0 x, 1 y, 2 z) of length n: dense products on the
+// matrix cores or the mixed-radix passes; false if neither takes it (hipFFT).
+// Measured alone on cubic grids, us a pass, dense / mixed radix:
+//   length   49          84         99         121          144         182         243          256
+//   y     4.0 / 6.0   5.2 / 8.5  7.5 / 18   11.0 / 10.0  15.3 / 35   29 / 103    62 / 232     78 / 129
+//   x     6.1 / 8.7   8.0 / 12   12 / 27    17.2 / 15.6  29 / 51     55 / 152   146 / 294    156 / 200
+//   z     4.2 / 4.9   6.4 / 6.8  7.7 / 15   11.1 / 11.5  22 / 30     39 / 89     94 / 149    132 / 116
+//   1/z   4.0 / 5.6   6.0 / 6.9  7.1 / 15   10.0 / 12.0  20 / 32     35 / 86     82 / 144    113 / 125
+// The mixed radix is the better one only where two radices make up the length
+// (16 lanes a line, so that its tiles are 8 complex columns wide) and the dense
+// product has grown: x and y from 100 up.  The dense z passes have no front
+// stage, so they stay ahead up to about 250.  A length with a factor above 13
+// has no mixed-radix form; dense, 61 takes 4.2 us (y), 137 16.5, 211 69, 307 220.
+static bool fft_plan(int n, int d, FftAxis& a) {
+    const bool smooth = fft_factor(n, a);
+    const bool two = smooth && a.lgP <= 4 && n >= 100;
+    a.dense = n <= kDftMaxLength && !(smooth && (d == 2 ? n > 250 : two));
+    // front radix of the dense x and y passes: the fewest matrix products, a point
+    // of the front stage counted as two
+    a.front = 1;
+    int best = 1 << 30;
+    for (int f : {1, 2, 3, 4}) {
+        if (n % f || n / f < 2) continue;
+        const int h = n / f / 2 + 1, cost = f * ((h + 15) / 16) * ((h + 3) / 4) + 2 * f;
+        if (cost < best) {
+            best = cost;
+            a.front = f;
+        }
+    }
+    return smooth || a.dense;
 }
 
 // Brick size along one grid axis for the spreading kernel: every brick at least
@@ -439,15 +474,19 @@ int elec_create(mbpol_context* ctx) {
     if (P.pme) {
         const size_t nreal = (size_t)grid[0] * grid[1] * grid[2];
         bool lds = true;
-        for (int d = 0; d < 3; ++d) lds = lds && fft_factor(grid[d], E->fft.ax[d]);
-        const char* force = std::getenv("MBPOL_HIP_PME_FFT");  // "hipfft" selects the library transforms
+        for (int d = 0; d < 3; ++d) lds = fft_plan(grid[d], d, E->fft.ax[d]) && lds;
+        // "hipfft" selects the library transforms, "radix" the mixed-radix passes where the length has them
+        const char* force = std::getenv("MBPOL_HIP_PME_FFT");
         if (force && std::string(force) == "hipfft") lds = false;
+        if (force && std::string(force) == "radix")
+            for (FftAxis& a : E->fft.ax) a.dense = a.dense && a.nfac == 0;
         E->lds_fft = lds;
         // z and y passes fused per x plane: faster alone, but a plane workgroup takes a
         // whole CU and stalls beside the short-range kernels on the second stream,
         // so the five single-axis passes are the default (MBPOL_HIP_PME_PLANES=1: planes)
         const char* planes = std::getenv("MBPOL_HIP_PME_PLANES");
-        E->plane_fft = lds && planes && std::string(planes) == "1" && fft_plane_ok(E->fft);
+        E->plane_fft = lds && planes && std::string(planes) == "1" && E->fft.ax[1].nfac > 0 && E->fft.ax[2].nfac > 0 &&
+                       fft_plane_ok(E->fft);
         const char* fuse = std::getenv("MBPOL_HIP_SPREAD_FUSED");
         E->fuse_spread = !(fuse && std::string(fuse) == "0");
         // half-spectrum rows: padded to 128 bytes for the LDS transforms, packed for hipFFT
@@ -476,7 +515,7 @@ int elec_create(mbpol_context* ctx) {
                 std::vector<double2> tw(m);
                 for (int t = 0; t < m; ++t) {
                     const long double a = 2.0L * 3.141592653589793238462643383279502884L * t / m;
-                    tw[t] = make_double2((double)cosl(a), (double)-sinl(a));
+                    tw[t] = 2 * t == m ? make_double2(-1.0, 0.0) : make_double2((double)cosl(a), (double)-sinl(a));
                 }
                 if (int e = up(ctx->stream, E->tw[d], tw)) return e;
                 E->fft.ax[d].tw = E->tw[d].as<double2>();

@@ -18,6 +18,8 @@ struct FftAxis {
     int lgP;
     int inplace;  // every stage has at most 2^lgP butterflies: stages run in place (one LDS buffer)
     const double2* tw;
+    int dense;  // the axis runs as dense products (kernels_dft.hip), after a front stage of radix `front`
+    int front;
 };
 
 struct PmeFft {
@@ -43,6 +45,17 @@ void launch_fft_x_conv(hipStream_t s, const PmeFft& F, double2* H, const double*
                        const int* stop = nullptr);
 void launch_fft_z_c2r(hipStream_t s, const PmeFft& F, const double2* H, double* real, const KEvents& ev,
                       const int* stop = nullptr);
+// the same passes as dense products on the FP64 matrix cores, for lengths up to kDftMaxLength (kernels_dft.hip)
+constexpr int kDftMaxLength = 512;
+void launch_dft_z_r2c(hipStream_t s, const PmeFft& F, const double* real, double2* H, const KEvents& ev,
+                      const int* stop);
+void launch_spread_dft_z_r2c(hipStream_t s, const PmeFft& F, const int* rowstart, const int* esite,
+                             const double* ecoef, const double* mu, double2* H, const KEvents& ev, const int* stop);
+void launch_dft_y(hipStream_t s, const PmeFft& F, double2* H, int inverse, const KEvents& ev, const int* stop);
+void launch_dft_x_conv(hipStream_t s, const PmeFft& F, double2* H, const double* influence, const KEvents& ev,
+                       const int* stop);
+void launch_dft_z_c2r(hipStream_t s, const PmeFft& F, const double2* H, double* real, const KEvents& ev,
+                      const int* stop);
 // z and y passes of one direction as one kernel per x plane (plane in LDS);
 // fft_plane_ok: the plane fits in LDS and every stage has at most one butterfly per thread
 bool fft_plane_ok(const PmeFft& F);

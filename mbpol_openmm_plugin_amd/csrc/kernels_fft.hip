@@ -19,48 +19,10 @@
 
 #include "device_common.h"
 #include "fft_kernels.h"
+#include "fft_roots.h"
 
 namespace mbpol {
 namespace {
-
-// cos / sin of 2 pi t / R, t < R
-template <int R>
-struct Roots;
-template <>
-struct Roots<2> {
-    static constexpr double c[2] = {1.0, -1.0};
-    static constexpr double s[2] = {0.0, 0.0};
-};
-template <>
-struct Roots<3> {
-    static constexpr double c[3] = {1.0, -0.5, -0.5};
-    static constexpr double s[3] = {0.0, 0.8660254037844386, -0.8660254037844386};
-};
-template <>
-struct Roots<4> {
-    static constexpr double c[4] = {1.0, 0.0, -1.0, 0.0};
-    static constexpr double s[4] = {0.0, 1.0, 0.0, -1.0};
-};
-template <>
-struct Roots<5> {
-    static constexpr double c[5] = {1.0, 0.30901699437494745, -0.8090169943749475, -0.8090169943749475, 0.30901699437494745};
-    static constexpr double s[5] = {0.0, 0.9510565162951535, 0.5877852522924731, -0.5877852522924731, -0.9510565162951535};
-};
-template <>
-struct Roots<7> {
-    static constexpr double c[7] = {1.0, 0.6234898018587335, -0.2225209339563144, -0.9009688679024191, -0.9009688679024191, -0.2225209339563144, 0.6234898018587335};
-    static constexpr double s[7] = {0.0, 0.7818314824680298, 0.9749279121818236, 0.4338837391175581, -0.4338837391175581, -0.9749279121818236, -0.7818314824680298};
-};
-template <>
-struct Roots<11> {
-    static constexpr double c[11] = {1.0, 0.8412535328311812, 0.41541501300188644, -0.14231483827328514, -0.6548607339452851, -0.9594929736144974, -0.9594929736144974, -0.6548607339452851, -0.14231483827328514, 0.41541501300188644, 0.8412535328311812};
-    static constexpr double s[11] = {0.0, 0.5406408174555976, 0.9096319953545183, 0.9898214418809327, 0.7557495743542583, 0.28173255684142967, -0.28173255684142967, -0.7557495743542583, -0.9898214418809327, -0.9096319953545183, -0.5406408174555976};
-};
-template <>
-struct Roots<13> {
-    static constexpr double c[13] = {1.0, 0.8854560256532099, 0.5680647467311558, 0.12053668025532305, -0.3546048870425356, -0.7485107481711011, -0.970941817426052, -0.970941817426052, -0.7485107481711011, -0.3546048870425356, 0.12053668025532305, 0.5680647467311558, 0.8854560256532099};
-    static constexpr double s[13] = {0.0, 0.46472317204376856, 0.8229838658936564, 0.992708874098054, 0.9350162426854148, 0.6631226582407952, 0.23931566428755777, -0.23931566428755777, -0.6631226582407952, -0.9350162426854148, -0.992708874098054, -0.8229838658936564, -0.46472317204376856};
-};
 
 // One radix-R Stockham step (stage with Ns = product of the earlier radices)
 // for butterfly j of a line of length N: inputs at j + r N/R, twiddle
@@ -806,29 +768,34 @@ static size_t lds_bytes(const FftAxis& a) {
 
 void launch_fft_z_r2c(hipStream_t s, const PmeFft& F, const double* real, double2* H, const KEvents& ev,
                       const int* stop) {
+    if (F.ax[2].dense) return launch_dft_z_r2c(s, F, real, H, ev, stop);
     const int nl = F.ax[0].n * F.ax[1].n, M = kFftThreads >> F.ax[2].lgP, Kh = F.ax[2].n / 2 + 1;
     MBPOL_FFT_LAUNCH(k_fft_z_r2c, F.ax[2], nblk(nl, M), kFftThreads, lds_bytes(F.ax[2]), s, real, H, nl, F.ax[2], Kh,
                      F.khp, stop)
 }
 void launch_spread_fft_z_r2c(hipStream_t s, const PmeFft& F, const int* rowstart, const int* esite,
                              const double* ecoef, const double* mu, double2* H, const KEvents& ev, const int* stop) {
+    if (F.ax[2].dense) return launch_spread_dft_z_r2c(s, F, rowstart, esite, ecoef, mu, H, ev, stop);
     const int nl = F.ax[0].n * F.ax[1].n, M = kFftThreads >> F.ax[2].lgP, Kh = F.ax[2].n / 2 + 1;
     MBPOL_FFT_LAUNCH(k_spread_fft_z_r2c, F.ax[2], nblk(nl, M), kFftThreads, lds_bytes(F.ax[2]), s, rowstart, esite,
                      ecoef, mu, H, nl, F.ax[2], Kh, F.khp, stop)
 }
 void launch_fft_y(hipStream_t s, const PmeFft& F, double2* H, int inverse, const KEvents& ev, const int* stop) {
+    if (F.ax[1].dense) return launch_dft_y(s, F, H, inverse, ev, stop);
     const int K0 = F.ax[0].n, K1 = F.ax[1].n, Kh = F.ax[2].n / 2 + 1, M = kFftThreads >> F.ax[1].lgP;
     MBPOL_FFT_LAUNCH(k_fft_y, F.ax[1], K0 * nblk(Kh, M), kFftThreads, lds_bytes(F.ax[1]), s, H, K1, Kh, F.khp, F.ax[1],
                      inverse, stop)
 }
 void launch_fft_x_conv(hipStream_t s, const PmeFft& F, double2* H, const double* influence, const KEvents& ev,
                        const int* stop) {
+    if (F.ax[0].dense) return launch_dft_x_conv(s, F, H, influence, ev, stop);
     const int K1 = F.ax[1].n, Kh = F.ax[2].n / 2 + 1, M = kFftThreads >> F.ax[0].lgP;
     MBPOL_FFT_LAUNCH(k_fft_x_conv, F.ax[0], K1 * nblk(Kh, M), kFftThreads, lds_bytes(F.ax[0]), s, H, influence, K1, Kh,
                      F.khp, F.ax[0], stop)
 }
 void launch_fft_z_c2r(hipStream_t s, const PmeFft& F, const double2* H, double* real, const KEvents& ev,
                       const int* stop) {
+    if (F.ax[2].dense) return launch_dft_z_c2r(s, F, H, real, ev, stop);
     const int nl = F.ax[0].n * F.ax[1].n, M = kFftThreads >> F.ax[2].lgP, Kh = F.ax[2].n / 2 + 1;
     MBPOL_FFT_LAUNCH(k_fft_z_c2r, F.ax[2], nblk(nl, M), kFftThreads, lds_bytes(F.ax[2]), s, H, real, nl, F.ax[2], Kh,
                      F.khp, stop)
