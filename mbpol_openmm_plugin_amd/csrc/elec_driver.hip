@@ -763,7 +763,7 @@ static int pme_grid(mbpol_context* ctx, int mode, const double* mu, const int* s
 // steps (a step that only returns costs ~8 launches, a read ~35 us).  With
 // timing on, or with hipFFT transforms (which cannot skip), one step per batch.
 static int solve_batch(const Elec* E, const mbpol_context* ctx, int batch) {
-    if (ctx->timer.enabled || !E->lds_fft) return 1;
+    if (ctx->timer.enabled || (E->P.pme && !E->lds_fft)) return 1;
     if (batch == 0) return std::max(1, E->last_iters);
     return 1 << std::min(batch - 1, 4);
 }
