@@ -84,7 +84,7 @@ struct DevBuf {
 struct CellGrid {
     ListGeom g{};
     int ncell = 0;
-    DevBuf cell_of, cell_count, cell_start, cell_fill, members;
+    DevBuf cell_of, cell_count, cell_start, cell_fill, cpos;  // cpos: positions and indices in cell order
 };
 
 // HIP-event timing of kernel groups on the context's stream.
@@ -181,7 +181,8 @@ struct mbpol_context {
     long long dimer_cap = 0;
     mbpol::DevBuf lo_count, lo_start, lower;
     int lower_cap = 0;
-    mbpol::DevBuf trip_count, trip_off, trips;
+    mbpol::DevBuf trip_count, trip_off, trips;  // counts and offsets per pair of the lower lists
+    mbpol::DevBuf trip_mol_off;                 // offsets per molecule (independent groups)
     long long trip_cap = 0;
     int lists_built = 0;        // lists built by this evaluation: 1 dimers, 2 trimers
     mbpol::DevBuf results_stage;  // energies and list lengths gathered for the one read-back (11 u64, every system)

@@ -92,17 +92,20 @@ void launch_scan_i64(hipStream_t s, const long long* in, long long* out, long lo
 // ---- kernels_lists.hip ----
 void launch_cell_count(hipStream_t s, int n, const int* idx, const double* pos, d3 L, int3 nc, int* cell_of,
                        int* cell_count);
-void launch_cell_fill(hipStream_t s, int n, const int* cell_of, const int* cell_start, int* cell_fill,
-                      int* cell_members);
+void launch_cell_fill(hipStream_t s, int n, const int* idx, const double* pos, const ListGeom& g, int phantoms,
+                      const int* cell_of, const int* cell_start, int* cell_fill, double4* cpos);
 void launch_dimer_pass(hipStream_t s, int n, const int* idx, const double* pos, ListGeom g, const int* cell_of,
-                       const int* cell_start, const int* cell_members, long long* count, const long long* offset,
+                       const int* cell_start, const double4* cpos, long long* count, const long long* offset,
                        int2* pairs, long long cap);
 void launch_lower_pass(hipStream_t s, int n, const int* idx, const double* pos, ListGeom g, const int* cell_of,
-                       const int* cell_start, const int* cell_members, int* count, const int* offset, int* lower,
+                       const int* cell_start, const double4* cpos, int* count, const int* offset, int2* lower,
                        int cap);
+// count / offset: lower_cap + 1 entries, one per pair (i, j) of the lower lists
 void launch_trimer_pass(hipStream_t s, int n, const int* idx, const double* pos, ListGeom g, const int* lo_start,
-                        const int* lower, int full_list, long long* count, const long long* offset, int* trip,
+                        const int2* lower, int full_list, long long* count, const long long* offset, int* trip,
                         int lower_cap, long long cap);
+// out[i] = off[min(start[i], limit)], i <= n
+void launch_offsets_of(hipStream_t s, int n, const int* start, int limit, const long long* off, long long* out);
 
 // ---- kernels_pip.hip (one object per body order and precision) ----
 // n: the list's capacity (grid size); ndev (optional): its length on the device (the kernels

@@ -427,7 +427,7 @@ static int setup_grid(mbpol_context* ctx, CellGrid& cg, int n, bool periodic, do
     HIP_TRY(cg.cell_count.ensure(sizeof(int) * (cg.ncell + 1)));
     HIP_TRY(cg.cell_start.ensure(sizeof(int) * (cg.ncell + 1)));
     HIP_TRY(cg.cell_fill.ensure(sizeof(int) * (cg.ncell + 1)));
-    HIP_TRY(cg.members.ensure(sizeof(int) * std::max(n, 1)));
+    HIP_TRY(cg.cpos.ensure(sizeof(double4) * std::max(n, 1)));
     return MBPOL_OK;
 }
 
@@ -486,15 +486,14 @@ static void apply_list_groups(mbpol_context* ctx) {
     }
 }
 
-static int bin_cells(mbpol_context* ctx, hipStream_t st, CellGrid& cg, int n, const int* idx) {
+// (the cell counters are cleared by the caller)
+static int bin_cells(mbpol_context* ctx, hipStream_t st, CellGrid& cg, int n, const int* idx, int phantoms) {
     if (!cg.g.use_cells) return MBPOL_OK;
-    launch_fill_zero(st, cg.cell_count.p, sizeof(int) * (cg.ncell + 1));
-    launch_fill_zero(st, cg.cell_fill.p, sizeof(int) * (cg.ncell + 1));
     launch_cell_count(st, n, idx, ctx->pos.as<double>(), cg.g.L, cg.g.nc, cg.cell_of.as<int>(),
                       cg.cell_count.as<int>());
     if (int e = scan_i32(ctx, cg.cell_count.as<int>(), cg.cell_start.as<int>(), cg.ncell + 1, st)) return e;
-    launch_cell_fill(st, n, cg.cell_of.as<int>(), cg.cell_start.as<int>(), cg.cell_fill.as<int>(),
-                     cg.members.as<int>());
+    launch_cell_fill(st, n, idx, ctx->pos.as<double>(), cg.g, phantoms, cg.cell_of.as<int>(), cg.cell_start.as<int>(),
+                     cg.cell_fill.as<int>(), cg.cpos.as<double4>());
     return MBPOL_OK;
 }
 
@@ -602,8 +601,7 @@ int mbpol_context_create(const mbpol_system* sys, int32_t precision, int32_t dev
     }
     if (n3 > 0) {
         if (int e = setup_grid(ctx, ctx->grid3, n3, sys->th_method == MBPOL_CUTOFF_PERIODIC, sys->th_cutoff)) return fail(e);
-        if (ctx->lo_count.ensure(sizeof(int) * (n3 + 1)) || ctx->lo_start.ensure(sizeof(int) * (n3 + 1)) ||
-            ctx->trip_count.ensure(sizeof(long long) * (n3 + 1)) || ctx->trip_off.ensure(sizeof(long long) * (n3 + 1)))
+        if (ctx->lo_count.ensure(sizeof(int) * (n3 + 1)) || ctx->lo_start.ensure(sizeof(int) * (n3 + 1)))
             return fail(set_error(MBPOL_ERR_HIP, "device allocation failed"));
     }
     apply_list_groups(ctx);
@@ -733,7 +731,7 @@ int mbpol_context_set_graph(mbpol_context* ctx, int32_t enabled) {
 }  // extern "C"
 
 // Build the dimer list and the trimer work list.  The list lengths stay on the
-// device (dimer_off[n2], lo_start[n3], trip_off[n3]): the fill passes write
+// device (dimer_off[n2], lo_start[n3], trip_off[lower_cap]): the fill passes write
 // what fits in the current capacities, the PIP kernels read the lengths, and
 // the host compares lengths and capacities after the evaluation (list_check),
 // growing the lists and running the evaluation again when one did not fit.
@@ -751,12 +749,20 @@ static int build_lists(mbpol_context* ctx, hipStream_t st, bool want2, bool want
         }
         return MBPOL_OK;
     };
+    {
+        FillList L(st);
+        for (CellGrid* g : {want2 ? &ctx->grid2 : nullptr, want3 ? &ctx->grid3 : nullptr})
+            if (g && g->g.use_cells) {
+                L.add(g->cell_count.p, sizeof(int) * (g->ncell + 1));
+                L.add(g->cell_fill.p, sizeof(int) * (g->ncell + 1));
+            }
+        L.launch();
+    }
     if (want2) {
         CellGrid& g = ctx->grid2;
-        if (int e = bin_cells(ctx, st, g, n2, ctx->tb_idx.as<int>())) return e;
-        launch_fill_zero(st, ctx->dimer_count.p, sizeof(long long) * (n2 + 1));
+        if (int e = bin_cells(ctx, st, g, n2, ctx->tb_idx.as<int>(), 0)) return e;
         launch_dimer_pass(st, n2, ctx->tb_idx.as<int>(), pos, g.g, g.cell_of.as<int>(), g.cell_start.as<int>(),
-                          g.members.as<int>(), ctx->dimer_count.as<long long>(), nullptr, nullptr, 0);
+                          g.cpos.as<double4>(), ctx->dimer_count.as<long long>(), nullptr, nullptr, 0);
         if (int e = scan_i64(ctx, ctx->dimer_count.as<long long>(), ctx->dimer_off.as<long long>(), n2 + 1, st)) return e;
         if (ctx->dimer_cap == 0) {  // first build: size the list
             HIP_TRY(hipMemcpyAsync(&hc[0], ctx->dimer_off.as<long long>() + n2, sizeof(long long),
@@ -765,38 +771,39 @@ static int build_lists(mbpol_context* ctx, hipStream_t st, bool want2, bool want
             if (int e = grow2(hc[0])) return e;
         }
         launch_dimer_pass(st, n2, ctx->tb_idx.as<int>(), pos, g.g, g.cell_of.as<int>(), g.cell_start.as<int>(),
-                          g.members.as<int>(), nullptr, ctx->dimer_off.as<long long>(), ctx->dimers.as<int2>(),
+                          g.cpos.as<double4>(), nullptr, ctx->dimer_off.as<long long>(), ctx->dimers.as<int2>(),
                           ctx->dimer_cap);
     }
     if (want3) {
         CellGrid& g = ctx->grid3;
-        if (int e = bin_cells(ctx, st, g, n3, ctx->th_idx.as<int>())) return e;
-        launch_fill_zero(st, ctx->lo_count.p, sizeof(int) * (n3 + 1));
+        if (int e = bin_cells(ctx, st, g, n3, ctx->th_idx.as<int>(), 1)) return e;
         launch_lower_pass(st, n3, ctx->th_idx.as<int>(), pos, g.g, g.cell_of.as<int>(), g.cell_start.as<int>(),
-                          g.members.as<int>(), ctx->lo_count.as<int>(), nullptr, nullptr, 0);
+                          g.cpos.as<double4>(), ctx->lo_count.as<int>(), nullptr, nullptr, 0);
         if (int e = scan_i32(ctx, ctx->lo_count.as<int>(), ctx->lo_start.as<int>(), n3 + 1, st)) return e;
         if (ctx->lower_cap == 0) {
             HIP_TRY(hipMemcpyAsync(&hc[1], ctx->lo_start.as<int>() + n3, sizeof(int), hipMemcpyDeviceToHost, st));
             HIP_TRY(hipStreamSynchronize(st));
             const int nl = (int)(reinterpret_cast<int*>(&hc[1])[0]);
-            HIP_TRY(ctx->lower.ensure(sizeof(int) * (nl + nl / 4 + 64)));
+            HIP_TRY(ctx->lower.ensure(sizeof(int2) * (nl + nl / 4 + 64)));
             ctx->lower_cap = nl + nl / 4 + 64;
         }
         launch_lower_pass(st, n3, ctx->th_idx.as<int>(), pos, g.g, g.cell_of.as<int>(), g.cell_start.as<int>(),
-                          g.members.as<int>(), nullptr, ctx->lo_start.as<int>(), ctx->lower.as<int>(), ctx->lower_cap);
-        launch_fill_zero(st, ctx->trip_count.p, sizeof(long long) * (n3 + 1));
-        launch_trimer_pass(st, n3, ctx->th_idx.as<int>(), pos, g.g, ctx->lo_start.as<int>(), ctx->lower.as<int>(),
+                          g.cpos.as<double4>(), nullptr, ctx->lo_start.as<int>(), ctx->lower.as<int2>(), ctx->lower_cap);
+        const size_t npair = (size_t)ctx->lower_cap + 1;  // one count per entry of the lower lists' capacity
+        HIP_TRY(ctx->trip_count.ensure(sizeof(long long) * npair));
+        HIP_TRY(ctx->trip_off.ensure(sizeof(long long) * npair));
+        launch_trimer_pass(st, n3, ctx->th_idx.as<int>(), pos, g.g, ctx->lo_start.as<int>(), ctx->lower.as<int2>(),
                            ctx->full_chain_list, ctx->trip_count.as<long long>(), nullptr, nullptr, ctx->lower_cap, 0);
-        if (int e = scan_i64(ctx, ctx->trip_count.as<long long>(), ctx->trip_off.as<long long>(), n3 + 1, st)) return e;
+        if (int e = scan_i64(ctx, ctx->trip_count.as<long long>(), ctx->trip_off.as<long long>(), (int)npair, st)) return e;
         if (ctx->trip_cap == 0) {
-            HIP_TRY(hipMemcpyAsync(&hc[2], ctx->trip_off.as<long long>() + n3, sizeof(long long), hipMemcpyDeviceToHost,
+            HIP_TRY(hipMemcpyAsync(&hc[2], ctx->trip_off.as<long long>() + ctx->lower_cap, sizeof(long long), hipMemcpyDeviceToHost,
                                    st));
             HIP_TRY(hipStreamSynchronize(st));
             const long long nt = hc[2];
             HIP_TRY(ctx->trips.ensure(sizeof(int) * 3 * (nt + nt / 4 + 64)));
             ctx->trip_cap = nt + nt / 4 + 64;
         }
-        launch_trimer_pass(st, n3, ctx->th_idx.as<int>(), pos, g.g, ctx->lo_start.as<int>(), ctx->lower.as<int>(),
+        launch_trimer_pass(st, n3, ctx->th_idx.as<int>(), pos, g.g, ctx->lo_start.as<int>(), ctx->lower.as<int2>(),
                            ctx->full_chain_list, nullptr, ctx->trip_off.as<long long>(), ctx->trips.as<int>(),
                            ctx->lower_cap, ctx->trip_cap);
     }
@@ -822,7 +829,7 @@ static int list_check(mbpol_context* ctx, bool& redo) {
     if (ctx->lists_built & 2) {
         const long long nl = hc[17], nt = hc[18];
         if (nl > ctx->lower_cap) {
-            HIP_TRY(ctx->lower.ensure(sizeof(int) * (nl + nl / 4 + 64)));
+            HIP_TRY(ctx->lower.ensure(sizeof(int2) * (nl + nl / 4 + 64)));
             ctx->lower_cap = (int)(nl + nl / 4 + 64);
             redo = true;  // the trimer list could not be built: its length is unknown
         } else if (nt > ctx->trip_cap) {
@@ -844,7 +851,7 @@ static int results_to_host(mbpol_context* ctx, hipStream_t st) {
     const bool l2 = ctx->lists_built & 1, l3 = ctx->lists_built & 2;
     u64* stage = ctx->results_stage.as<u64>();
     launch_collect_results(st, ctx->energy_fx.as<u64>(), l2 ? ctx->dimer_off.as<long long>() + n2 : nullptr,
-                           l3 ? ctx->lo_start.as<int>() + n3 : nullptr, l3 ? ctx->trip_off.as<long long>() + n3 : nullptr,
+                           l3 ? ctx->lo_start.as<int>() + n3 : nullptr, l3 ? ctx->trip_off.as<long long>() + ctx->lower_cap : nullptr,
                            stage);
     HIP_TRY(hipMemcpyAsync(static_cast<u64*>(ctx->h_counts) + 8, stage, sizeof(u64) * 11, hipMemcpyDeviceToHost, st));
     return MBPOL_OK;
@@ -908,7 +915,7 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
             const int per = s.th_method == MBPOL_CUTOFF_PERIODIC;
             const KEvents ev = timer_kernel(ctx, T_THREEBODY);
             const long long nt = ctx->trip_cap;
-            const long long* ntd = ctx->trip_off.as<long long>() + (int)s.th_idx.size() / 3;  // list length (device)
+            const long long* ntd = ctx->trip_off.as<long long>() + ctx->lower_cap;  // list length (device)
             const int* tr = ctx->trips.as<int>();
             const int* ti = ctx->th_idx.as<int>();
             const int cap = ctx->pip3_blocks;
@@ -919,9 +926,14 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
             else
                 launch_threebody_orbit_f64(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2, ev, eu3, cap);
             timer_kernel_done(ctx, T_THREEBODY, ev);
-            if (G)
-                launch_group_sums(sr, G, ctx->g_wstart.as<int>(), 0, ctx->trip_off.as<long long>(), eu3, EG, 2,
+            if (G) {
+                const int n3 = (int)s.th_idx.size() / 3;
+                HIP_TRY(ctx->trip_mol_off.ensure(sizeof(long long) * (n3 + 1)));
+                launch_offsets_of(sr, n3, ctx->lo_start.as<int>(), ctx->lower_cap, ctx->trip_off.as<long long>(),
+                                  ctx->trip_mol_off.as<long long>());
+                launch_group_sums(sr, G, ctx->g_wstart.as<int>(), 0, ctx->trip_mol_off.as<long long>(), eu3, EG, 2,
                                   ctx->trip_cap);
+            }
         }
         return MBPOL_OK;
     };
