@@ -416,7 +416,15 @@ def main():
                   'constexpr unsigned %s_step_mask = 0x%xu;' % (prefix, mask),
                   'constexpr int %s_step_a[%d] = {%s};' % (prefix, nvar, ', '.join(str(v) for v in a)),
                   'constexpr int %s_step_b[%d] = {%s};' % (prefix, nvar, ', '.join(str(v) for v in b)),
-                  'constexpr int %s_orbit_ncoef = %d;' % (prefix, len(table))]
+                  'constexpr int %s_orbit_ncoef = %d;' % (prefix, len(table)),
+                  '// labelling of the registers before pass k (and after the last): y[m] = x[%s_label[%d k + m]]'
+                  % (prefix, nvar),
+                  '__constant__ int %s_label[%d] = {' % (prefix, nvar * (len(group) + 1))]
+        label = tuple(range(nvar))
+        for k in range(len(group) + 1):
+            parts.append('    ' + ', '.join(str(v) for v in label) + ',')
+            label = compose(label, a if (mask >> k) & 1 else b)
+        parts.append('};')
         for typ, suf in (('double', 'f64'), ('float', 'f32')):
             parts.append('__constant__ %s %s_orbit_coef_%s[%d] = {' % (typ, prefix, suf, len(table)))
             for i in range(0, len(table), 4):

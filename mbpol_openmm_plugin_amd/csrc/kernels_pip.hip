@@ -13,6 +13,9 @@
 //   -DPIP_BODY=2|3  -DPIP_REAL=float|double
 // with -DPIP_ORBIT=1 the polynomial is evaluated through the relabelling group
 // of the dimer or trimer (pip_orbit_loop.h) instead of term by term.
+#include <algorithm>
+#include <type_traits>
+
 #include "device_common.h"
 // an empty asm that re-defines a variable in its register: no instruction
 #define PIP_FENCE(v) asm volatile("" : "+v"(v))
@@ -25,13 +28,6 @@
 #else
 #include "pip_eval_gen.h"
 #endif
-// Register budget of the 3-body kernel, as waves per SIMD (-DPIP3_WAVES=n)
-#if defined(PIP3_WAVES) && PIP3_WAVES > 1
-#define PIP3_OCCUPANCY __attribute__((amdgpu_waves_per_eu(PIP3_WAVES)))
-#else
-#define PIP3_OCCUPANCY
-#endif
-
 #ifndef PIP_BODY
 #error "PIP_BODY must be 2 or 3"
 #endif
@@ -45,7 +41,29 @@ using namespace mbpol_params;
 typedef PIP_REAL real;
 typedef v3<real> vr;
 
+// image_to by products with 1/L: the image index differs from the one the quotient
+// gives only where a separation is within rounding of half the box, at or beyond
+// every cutoff, where the switches are zero
+__device__ __forceinline__ d3 image_near(const d3& ref, const d3& p, const d3& L, const d3& iL) {
+    return d3{p.x + L.x * floor((ref.x - p.x) * iL.x + 0.5), p.y + L.y * floor((ref.y - p.y) * iL.y + 0.5),
+              p.z + L.z * floor((ref.z - p.z) * iL.z + 0.5)};
+}
+
 __device__ __forceinline__ vr rel(const d3& p, const d3& o) { return vr((real)(p.x - o.x), (real)(p.y - o.y), (real)(p.z - o.z)); }
+
+#if PIP_ORBIT
+// Forces of one molecule {idx[3 mol ..]} added by the lane that holds its run's sums.
+__device__ __forceinline__ void add_molecule(u64* __restrict__ force, const int* __restrict__ idx, long long mol,
+                                             bool last, const u64 (&f)[9]) {
+    if (!last || mol < 0) return;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const int a = idx[3 * mol + q];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) atomicAdd(&force[3 * a + d], f[3 * q + d]);
+    }
+}
+#endif
 
 #if PIP_BODY == 2
 // ---------------------------------------------------------------------------
@@ -59,7 +77,7 @@ struct Var2 {
 };
 // the 31 variables in reference order (:170-207)
 #define V2(a, b, c, k, r) {a, b, c, k, r}
-__device__ __forceinline__ Var2 var2(int n) {
+__host__ __device__ constexpr Var2 var2(int n) {
     const double di = tb_d0_intra, de = tb_d0_inter;
     switch (n) {
         case 0: return V2(1, 2, 0, tb_k_HH_intra, di);
@@ -98,10 +116,11 @@ __device__ __forceinline__ Var2 var2(int n) {
 #undef V2
 
 // extra points of one monomer (mbpol_2body_constants.cpp:62-76)
-__device__ __forceinline__ void extra_points(const vr& O, const vr& H1, const vr& H2, vr& x1, vr& x2) {
-    const vr oh1 = H1 - O, oh2 = H2 - O;
-    const vr in_plane = O + (oh1 + oh2) * (real)(0.5 * tb_in_plane_gamma);
-    const vr out_of_plane = oh1.cross(oh2) * (real)tb_out_of_plane_gamma;
+template <typename T>
+__device__ __forceinline__ void extra_points(const v3<T>& O, const v3<T>& H1, const v3<T>& H2, v3<T>& x1, v3<T>& x2) {
+    const v3<T> oh1 = H1 - O, oh2 = H2 - O;
+    const v3<T> in_plane = O + (oh1 + oh2) * (T)(0.5 * tb_in_plane_gamma);
+    const v3<T> out_of_plane = oh1.cross(oh2) * (T)tb_out_of_plane_gamma;
     x1 = in_plane + out_of_plane;
     x2 = in_plane - out_of_plane;
 }
@@ -141,11 +160,12 @@ __device__ __forceinline__ bool dimer_geometry(long long t, const int2* __restri
         P[q] = d3{p.x * 10., p.y * 10., p.z * 10.};
     }
     if (periodic) {  // imageMolecules (MBPolReferenceTwoBodyForce.cpp:78-100)
-        P[1] = image_to(P[0], P[1], boxA);
-        P[2] = image_to(P[0], P[2], boxA);
-        P[3] = image_to(P[0], P[3], boxA);
-        P[4] = image_to(P[3], P[4], boxA);
-        P[5] = image_to(P[3], P[5], boxA);
+        const d3 iL{1.0 / boxA.x, 1.0 / boxA.y, 1.0 / boxA.z};
+        P[1] = image_near(P[0], P[1], boxA, iL);
+        P[2] = image_near(P[0], P[2], boxA, iL);
+        P[3] = image_near(P[0], P[3], boxA, iL);
+        P[4] = image_near(P[3], P[4], boxA, iL);
+        P[5] = image_near(P[3], P[5], boxA, iL);
     }
     dOO = d3{P[0].x - P[3].x, P[0].y - P[3].y, P[0].z - P[3].z};
     rOO = sqrt(dOO.x * dOO.x + dOO.y * dOO.y + dOO.z * dOO.z);
@@ -157,6 +177,99 @@ __device__ __forceinline__ bool dimer_geometry(long long t, const int2* __restri
     return true;
 }
 
+// switch and its derivative (mbpol_2body_constants.cpp:98-111), FP64
+__device__ __forceinline__ void switch2(double rOO, double& sw, double& gsw) {
+    if (rOO > tb_r2i) {
+        constexpr double t1 = 1.0 / (tb_r2f - tb_r2i);
+        double sn, cs;
+        sincospi((rOO - tb_r2i) * t1, &sn, &cs);  // the argument in units of pi: no range reduction
+        gsw = -sn * (0.5 * M_PI * t1);
+        sw = (1.0 + cs) / 2.0;
+    } else {
+        sw = 1.0;
+        gsw = 0.0;
+    }
+}
+
+#if PIP_ORBIT
+typedef v3<double> vd;
+// the ten points of dimer t relative to Oa, Angstrom; whether it contributes
+__device__ __forceinline__ bool unit_geometry(long long t, const int2* __restrict__ pairs, const int* __restrict__ idx,
+                                              const double* __restrict__ pos, int periodic, const d3& box, vd (&R)[10]) {
+    const int2 pr = pairs[t];
+    d3 P[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+        const d3 p = load_d3(pos, idx[3 * (q < 3 ? pr.x : pr.y) + q % 3]);
+        P[q] = d3{p.x * 10., p.y * 10., p.z * 10.};
+    }
+    if (periodic) {  // imageMolecules (MBPolReferenceTwoBodyForce.cpp:78-100)
+        const d3 L{box.x * 10., box.y * 10., box.z * 10.}, iL{1.0 / L.x, 1.0 / L.y, 1.0 / L.z};
+        P[1] = image_near(P[0], P[1], L, iL);
+        P[2] = image_near(P[0], P[2], L, iL);
+        P[3] = image_near(P[0], P[3], L, iL);
+        P[4] = image_near(P[3], P[4], L, iL);
+        P[5] = image_near(P[3], P[5], L, iL);
+    }
+#pragma unroll
+    for (int q = 0; q < 6; ++q) R[q] = vd(P[q].x - P[0].x, P[q].y - P[0].y, P[q].z - P[0].z);
+    extra_points(R[0], R[1], R[2], R[6], R[7]);
+    extra_points(R[3], R[4], R[5], R[8], R[9]);
+    const double r = sqrt(R[3].dot(R[3]));
+    return r <= tb_r2f && r >= 2.;
+}
+
+__device__ __forceinline__ PIP_CONST_PTR(int) label_table() { return (PIP_CONST_PTR(int))pip2b_label; }
+template <typename T>
+__device__ __forceinline__ T passes(T (&x)[31], T (&g)[31], int k0, int k1) {
+    return pip2b_orbit_passes<T>(x, g, k0, k1);
+}
+
+// step 5: forces of molecule `part` (0, 1) or the energy (2)
+__device__ __forceinline__ void unit_end(int part, bool on, long long t, bool in, double E, const double (&rs)[30][64],
+                                         const real (&fs)[30][64], const int2* __restrict__ pairs,
+                                         const int* __restrict__ idx, u64* __restrict__ force,
+                                         u64* __restrict__ energy, double* __restrict__ eunit, int lane) {
+    const vd b(rs[9][lane], rs[10][lane], rs[11][lane]);  // Oa -> Ob
+    double sw = 0.0, gsw = 0.0;
+    const double r = sqrt(b.dot(b));
+    if (on) switch2(r, sw, gsw);
+    if (part == 2) {
+        const double e = on ? sw * E * cal2joule : 0.0;
+        if (eunit && in) eunit[t] = e;
+        add_energy(energy, e);
+        return;
+    }
+    u64 f[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    long long key = in ? (long long)(part ? pairs[t].y : pairs[t].x) : -1;
+    if (on) {
+        auto point = [&](const auto& v, int q) { return vr((real)v[3 * q][lane], (real)v[3 * q + 1][lane], (real)v[3 * q + 2][lane]); };
+        const int o = 3 * part, x = 6 + 2 * part;
+        vr F[3] = {point(fs, o), point(fs, o + 1), point(fs, o + 2)};
+        extra_grads(point(rs, o), point(rs, o + 1), point(rs, o + 2), point(fs, x), point(fs, x + 1), F[0], F[1], F[2]);
+        const double s = sw * cal2joule * -10.;
+        // of the switch, on the oxygens along Oa - Ob
+        const double gq = gsw * E / r * cal2joule * (part ? -10. : 10.);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            double fx = (double)F[q].x * s, fy = (double)F[q].y * s, fz = (double)F[q].z * s;
+            if (q == 0) {
+                fx += gq * b.x;
+                fy += gq * b.y;
+                fz += gq * b.z;
+            }
+            f[3 * q] = to_fix(fx);
+            f[3 * q + 1] = to_fix(fy);
+            f[3 * q + 2] = to_fix(fz);
+        }
+    }
+    // the first molecule's forces over the wave's runs of dimers that share it, the second's after a sort
+    const bool last = part == 0 ? wave_run_sum(key, f) : wave_sorted_run_sum(key, f);
+    add_molecule(force, idx, key, last, f);
+}
+#endif
+
+#if !PIP_ORBIT
 __global__ void __launch_bounds__(64) k_twobody(long long np, const long long* __restrict__ ndev,
                                                 const int2* __restrict__ pairs, const int* __restrict__ idx,
                                                 const double* __restrict__ pos, int periodic, d3 boxA,
@@ -188,11 +301,7 @@ __global__ void __launch_bounds__(64) k_twobody(long long np, const long long* _
                 const real e = exp_t<real>((real)v.k * ((real)v.r0 - r));
                 x[n] = v.coul ? e / r : e;
             }
-#if PIP_ORBIT
-            real Ep = pip2b_orbit_eval<real>(x, g);
-#else
             real Ep = pip2b_eval<real>(x, g);
-#endif
             // Only t, Ep and g stay live across the polynomial: the geometry is
             // reloaded from memory (the opaque copy of t keeps the compiler from
             // holding the first loads in registers through the polynomial).
@@ -225,17 +334,8 @@ __global__ void __launch_bounds__(64) k_twobody(long long np, const long long* _
             }
             extra_grads(R[0], R[1], R[2], F[6], F[7], F[0], F[1], F[2]);
             extra_grads(R[3], R[4], R[5], F[8], F[9], F[3], F[4], F[5]);
-            // switch (mbpol_2body_constants.cpp:98-111), FP64
             double sw, gsw;
-            if (rOO > tb_r2i) {
-                const double t1 = M_PI / (tb_r2f - tb_r2i);
-                const double xs = (rOO - tb_r2i) * t1;
-                gsw = -sin(xs) * t1 / 2.0;
-                sw = (1.0 + cos(xs)) / 2.0;
-            } else {
-                sw = 1.0;
-                gsw = 0.0;
-            }
+            switch2(rOO, sw, gsw);
             const double s = sw * cal2joule * -10.;
             const double gs = gsw * (double)Ep / rOO * cal2joule * -10.;
 #pragma unroll
@@ -275,6 +375,7 @@ __global__ void __launch_bounds__(64) k_twobody(long long np, const long long* _
         add_energy(energy, e_out);
     }
 }
+#endif
 
 #else
 // ---------------------------------------------------------------------------
@@ -282,11 +383,11 @@ __global__ void __launch_bounds__(64) k_twobody(long long np, const long long* _
 // Points (nm, relative to Oa): 0 Oa 1 Ha1 2 Ha2 3 Ob 4 Hb1 5 Hb2 6 Oc 7 Hc1 8 Hc2.
 // ---------------------------------------------------------------------------
 struct Var3 {
-    int a, b;
+    int a, b, coul;
     double k, r0;
 };
-#define V3(a, b, k, r) {a, b, k, r}
-__device__ __forceinline__ Var3 var3(int n) {
+#define V3(a, b, k, r) {a, b, 0, k, r}
+__host__ __device__ constexpr Var3 var3(int n) {
     switch (n) {  // reference order (:170-206)
         case 0: return V3(1, 2, th_kHH_intra, th_dHH_intra);
         case 1: return V3(4, 5, th_kHH_intra, th_dHH_intra);
@@ -331,10 +432,11 @@ __device__ __forceinline__ Var3 var3(int n) {
 __device__ __forceinline__ double switch3(double r, double& g) {  // (:103-120)
     if (r > th_r3f) { g = 0.0; return 0.0; }
     if (r > th_r3i) {
-        const double t1 = M_PI / (th_r3f - th_r3i);
-        const double x = (r - th_r3i) * t1;
-        g = -sin(x) * t1 / 2.0;
-        return (1.0 + cos(x)) / 2.0;
+        constexpr double t1 = 1.0 / (th_r3f - th_r3i);
+        double sn, cs;
+        sincospi((r - th_r3i) * t1, &sn, &cs);  // the argument in units of pi: no range reduction
+        g = -sn * (0.5 * M_PI * t1);
+        return (1.0 + cs) / 2.0;
     }
     g = 0.0;
     return 1.0;
@@ -356,14 +458,15 @@ __device__ __forceinline__ bool trimer_geometry(long long t, const int* __restri
 #pragma unroll
     for (int q = 0; q < 9; ++q) P[q] = load_d3(pos, at[q]);
     if (periodic) {  // imageMolecules in nm (MBPolReferenceTwoBodyForce.cpp:78-109)
-        P[1] = image_to(P[0], P[1], box);
-        P[2] = image_to(P[0], P[2], box);
-        P[3] = image_to(P[0], P[3], box);
-        P[4] = image_to(P[3], P[4], box);
-        P[5] = image_to(P[3], P[5], box);
-        P[6] = image_to(P[0], P[6], box);
-        P[7] = image_to(P[6], P[7], box);
-        P[8] = image_to(P[6], P[8], box);
+        const d3 iL{1.0 / box.x, 1.0 / box.y, 1.0 / box.z};
+        P[1] = image_near(P[0], P[1], box, iL);
+        P[2] = image_near(P[0], P[2], box, iL);
+        P[3] = image_near(P[0], P[3], box, iL);
+        P[4] = image_near(P[3], P[4], box, iL);
+        P[5] = image_near(P[3], P[5], box, iL);
+        P[6] = image_near(P[0], P[6], box, iL);
+        P[7] = image_near(P[6], P[7], box, iL);
+        P[8] = image_near(P[6], P[8], box, iL);
     }
     roo[0] = d3{(P[0].x - P[3].x) * 10., (P[0].y - P[3].y) * 10., (P[0].z - P[3].z) * 10.};  // ab
     roo[1] = d3{(P[0].x - P[6].x) * 10., (P[0].y - P[6].y) * 10., (P[0].z - P[6].z) * 10.};  // ac
@@ -380,7 +483,90 @@ __device__ __forceinline__ bool trimer_geometry(long long t, const int* __restri
     return true;
 }
 
-__global__ void __launch_bounds__(64) PIP3_OCCUPANCY k_threebody(long long nt, const long long* __restrict__ ndev,
+#if PIP_ORBIT
+typedef v3<double> vd;
+// the nine points of trimer t relative to Oa, Angstrom; whether it contributes
+__device__ __forceinline__ bool unit_geometry(long long t, const int* __restrict__ trip, const int* __restrict__ idx,
+                                              const double* __restrict__ pos, int periodic, const d3& box, vd (&R)[9]) {
+    d3 P[9];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) P[q] = load_d3(pos, idx[3 * trip[3 * t + q / 3] + q % 3]);
+    if (periodic) {  // imageMolecules in nm (MBPolReferenceTwoBodyForce.cpp:78-109)
+        const d3 iL{1.0 / box.x, 1.0 / box.y, 1.0 / box.z};
+        P[1] = image_near(P[0], P[1], box, iL);
+        P[2] = image_near(P[0], P[2], box, iL);
+        P[3] = image_near(P[0], P[3], box, iL);
+        P[4] = image_near(P[3], P[4], box, iL);
+        P[5] = image_near(P[3], P[5], box, iL);
+        P[6] = image_near(P[0], P[6], box, iL);
+        P[7] = image_near(P[6], P[7], box, iL);
+        P[8] = image_near(P[6], P[8], box, iL);
+    }
+#pragma unroll
+    for (int q = 0; q < 9; ++q) R[q] = vd((P[q].x - P[0].x) * 10., (P[q].y - P[0].y) * 10., (P[q].z - P[0].z) * 10.);
+    const vd bc = R[3] - R[6];
+    // nothing below 2 Angstrom (:160-163)
+    return !(R[3].dot(R[3]) < 4. || R[6].dot(R[6]) < 4. || bc.dot(bc) < 4.);
+}
+
+__device__ __forceinline__ PIP_CONST_PTR(int) label_table() { return (PIP_CONST_PTR(int))pip3b_label; }
+template <typename T>
+__device__ __forceinline__ T passes(T (&x)[36], T (&g)[36], int k0, int k1) {
+    return pip3b_orbit_passes<T>(x, g, k0, k1);
+}
+
+// step 5: forces of molecule `part` (0 .. 2) or the energy (3)
+__device__ __forceinline__ void unit_end(int part, bool on, long long t, bool in, double E, const double (&rs)[27][64],
+                                         const real (&fs)[27][64], const int* __restrict__ trip,
+                                         const int* __restrict__ idx, u64* __restrict__ force,
+                                         u64* __restrict__ energy, double* __restrict__ eunit, int lane) {
+    const vd b(rs[9][lane], rs[10][lane], rs[11][lane]), c(rs[18][lane], rs[19][lane], rs[20][lane]), bc = b - c;
+    double sab = 0, sac = 0, sbc = 0, gab = 0, gac = 0, gbc = 0;
+    const double rab = sqrt(b.dot(b)), rac = sqrt(c.dot(c)), rbc = sqrt(bc.dot(bc));
+    if (on) {
+        sab = switch3(rab, gab);
+        sac = switch3(rac, gac);
+        sbc = switch3(rbc, gbc);
+    }
+    const double s = sab * sac + sab * sbc + sac * sbc;
+    if (part == 3) {
+        const double e = on ? E * s * cal2joule : 0.0;
+        if (eunit && in) eunit[t] = e;
+        add_energy(energy, e);
+        return;
+    }
+    u64 f[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    long long key = in ? (long long)trip[3 * t + part] : -1;
+    if (on) {
+        const double fsc = s * cal2joule * 10. * -1, u = cal2joule * -nm_to_A;
+        gab *= (sac + sbc) * E / rab;
+        gac *= (sab + sbc) * E / rac;
+        gbc *= (sab + sac) * E / rbc;
+        // of the switches, on the oxygens along Oa - Ob = -b, Oa - Oc = -c, Ob - Oc = bc
+        const vd w = part == 0 ? b * -gab - c * gac : part == 1 ? bc * gbc + b * gab : c * gac - bc * gbc;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const int p = 3 * (3 * part + q);
+            double fx = (double)fs[p][lane] * fsc, fy = (double)fs[p + 1][lane] * fsc, fz = (double)fs[p + 2][lane] * fsc;
+            if (q == 0) {
+                fx += w.x * u;
+                fy += w.y * u;
+                fz += w.z * u;
+            }
+            f[3 * q] = to_fix(fx);
+            f[3 * q + 1] = to_fix(fy);
+            f[3 * q + 2] = to_fix(fz);
+        }
+    }
+    // the list is ordered by first, then second molecule: their forces are summed over the wave's runs of
+    // trimers that share them, the third's after a sort by molecule
+    const bool last = part < 2 ? wave_run_sum(key, f) : wave_sorted_run_sum(key, f);
+    add_molecule(force, idx, key, last, f);
+}
+#endif
+
+#if !PIP_ORBIT
+__global__ void __launch_bounds__(64) k_threebody(long long nt, const long long* __restrict__ ndev,
                                                                  const int* __restrict__ trip,
                                                                  const int* __restrict__ idx,
                                                                  const double* __restrict__ pos, int periodic, d3 box,
@@ -414,11 +600,7 @@ __global__ void __launch_bounds__(64) PIP3_OCCUPANCY k_threebody(long long nt, c
                 const real r = sqrt(d.dot(d));
                 x[n] = exp_t<real>(-(real)v.k * (r - (real)v.r0));
             }
-#if PIP_ORBIT
-            real Ep = pip3b_orbit_eval<real>(x, g);
-#else
             real Ep = pip3b_eval<real>(x, g);
-#endif
             // Only t, Ep and g stay live across the polynomial; the geometry is
             // reloaded (through an opaque copy of t, so that the first loads are
             // not kept in registers).
@@ -512,6 +694,177 @@ __global__ void __launch_bounds__(64) PIP3_OCCUPANCY k_threebody(long long nt, c
     }
 }
 #endif
+#endif
+
+#if PIP_ORBIT
+// ---------------------------------------------------------------------------
+// The polynomial through the unit's relabelling group: 64 dimers (trimers) a
+// block, the 8 (24) passes shared out among its 4 waves -- for a short list among
+// the 4 Q waves of Q blocks.
+//   1. wave 0 reads the geometry into LDS;
+//   2. the waves compute the variables (LDS);
+//   3. each wave takes them in the labelling its passes start from, runs its
+//      passes, and adds its gradient to the block's in the original labelling,
+//      one wave after the other: the sums do not depend on scheduling;
+//   4. the waves take the points in turn for the chain rule;
+//   5. wave m sums and adds the forces of molecule m, the wave after them the energy.
+// Steps 2 and 4 are rolled loops over tables of the variables, so that a unit's
+// code outside the passes is short and, for a short list, not fetched in vain.
+//
+// What bounds it: FP64 issue.  A wave alone on its SIMD issues one instruction in
+// 4.9 cycles, two one in 4.3 between them, and a pass is 4200 (3-body) or 4600
+// (2-body) instructions.  A long list fills two waves a SIMD, which 256 registers
+// allow; a short one lasts as long as one wave's share of the passes, so it is cut
+// finer until the waves would meet on a SIMD again (8 waves in one block on one CU
+// gained nothing over 4).  One wave per unit through all passes (2-body: term by
+// term) took, against this: 101 trimers 207 / 42 us, 13,641 238 / 101, 139,535
+// 566 / 450; 91 dimers 93 / 32, 4612 93 / 47, 42,250 105 / 83.
+// ---------------------------------------------------------------------------
+#if PIP_BODY == 2
+constexpr int kPoints = 10, kVars = 31, kMols = 2, kPassAll = pip2b_npass;
+typedef Var2 Var;
+typedef int2 Unit;
+__host__ __device__ constexpr Var var_of(int n) { return var2(n); }
+// points of molecule m: its atoms, then its extra points
+__device__ __forceinline__ int molecule_of(const Unit* list, long long t, int m) { return m ? list[t].y : list[t].x; }
+#else
+constexpr int kPoints = 9, kVars = 36, kMols = 3, kPassAll = pip3b_npass;
+typedef Var3 Var;
+typedef int Unit;
+__host__ __device__ constexpr Var var_of(int n) { return var3(n); }
+__device__ __forceinline__ int molecule_of(const Unit* list, long long t, int m) { return list[3 * t + m]; }
+#endif
+// the variables, and for every point the variables it enters with the point at the other end
+struct Partner {
+    int n, other, coul, pad;
+    double k;
+};
+struct PipTables {
+    Var var[kVars];
+    Partner with[kPoints][kPoints];
+    int count[kPoints];
+};
+constexpr PipTables make_tables() {
+    PipTables t{};
+    for (int n = 0; n < kVars; ++n) {
+        t.var[n] = var_of(n);
+        const int a = t.var[n].a, b = t.var[n].b;
+        t.with[a][t.count[a]++] = Partner{n, b, t.var[n].coul, 0, t.var[n].k};
+        t.with[b][t.count[b]++] = Partner{n, a, t.var[n].coul, 0, t.var[n].k};
+    }
+    return t;
+}
+__constant__ PipTables pip_tables = make_tables();
+
+__device__ __forceinline__ double rsqrt_pip(double v) { return rsqrt(v); }
+__device__ __forceinline__ float rsqrt_pip(float v) { return 1.0f / sqrtf(v); }
+
+constexpr int P = 4;  // waves of a block
+
+__global__ void __launch_bounds__(64 * P) __attribute__((amdgpu_waves_per_eu(2)))
+k_pip_split(int parts, long long nu, const long long* __restrict__ ndev, const Unit* __restrict__ list,
+            const int* __restrict__ idx, const double* __restrict__ pos, int periodic, d3 box,
+            u64* __restrict__ force, u64* __restrict__ energy, double* __restrict__ eunit) {
+    constexpr int N = kVars;
+    static_assert(P > kMols, "a wave for each part of step 5");
+    __shared__ double rs[kPoints * 3][64];          // points relative to the first oxygen, Angstrom
+    __shared__ real xs[N][64], gs[N][64], es[P][64];  // variables, gradient, energies of the waves' passes
+    __shared__ real fs[kPoints * 3][64];            // minus the gradient on the points (before switch and units)
+    __shared__ int ons[64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    PIP_CONST_PTR(PipTables) tab = (PIP_CONST_PTR(PipTables))&pip_tables;
+    if (ndev) nu = min(nu, *ndev);
+    const int part = blockIdx.x % parts, npass = kPassAll / (P * parts), k0 = (part * P + wave) * npass;
+    for (long long t0 = (long long)(blockIdx.x / parts) * 64; t0 < nu; t0 += (long long)(gridDim.x / parts) * 64) {
+        const long long t = t0 + lane;
+        if (wave == 0) {
+            bool on = false;
+            if (t < nu) {
+                vd R[kPoints];
+                on = unit_geometry(t, list, idx, pos, periodic, box, R);
+                if (on) {
+#pragma unroll
+                    for (int q = 0; q < kPoints; ++q) {
+                        rs[3 * q][lane] = R[q].x;
+                        rs[3 * q + 1][lane] = R[q].y;
+                        rs[3 * q + 2][lane] = R[q].z;
+                    }
+                }
+            }
+            if (!on) {  // any points apart: the results are not used
+#pragma unroll
+                for (int q = 0; q < kPoints; ++q) rs[3 * q][lane] = rs[3 * q + 1][lane] = rs[3 * q + 2][lane] = (double)q;
+            }
+            ons[lane] = on;
+        }
+        __syncthreads();
+        const bool on = ons[lane];
+#pragma unroll 3
+        for (int n = wave; n < N; n += P) {
+            const int a = 3 * tab->var[n].a, b = 3 * tab->var[n].b;
+            const vr d((real)(rs[a][lane] - rs[b][lane]), (real)(rs[a + 1][lane] - rs[b + 1][lane]),
+                       (real)(rs[a + 2][lane] - rs[b + 2][lane]));
+            const real r = sqrt(d.dot(d));
+            const real e = exp_t<real>((real)tab->var[n].k * ((real)tab->var[n].r0 - r));
+            xs[n][lane] = tab->var[n].coul ? e / r : e;
+        }
+        __syncthreads();
+        {
+            PIP_CONST_PTR(int) from = label_table() + N * k0;
+            real x[N], g[N];
+#pragma unroll
+            for (int m = 0; m < N; ++m) x[m] = xs[from[m]][lane];
+            real e = 0;
+#if PIP_BODY == 3
+            if (k0 == 0) {  // R: this wave starts from the original labelling
+                e = pip3b_rest<real>(x, g);
+            } else
+#endif
+            {
+#pragma unroll
+                for (int m = 0; m < N; ++m) g[m] = 0;
+            }
+            e += passes<real>(x, g, k0, k0 + npass);
+            es[wave][lane] = e;
+            PIP_CONST_PTR(int) to = label_table() + N * (k0 + npass);
+            PIP_OPAQUE_PTR(to);  // read after the passes
+            for (int w = 0; w < P; ++w) {
+                if (w == wave) {
+#pragma unroll
+                    for (int m = 0; m < N; ++m) {
+                        const int i = to[m];
+                        gs[i][lane] = w == 0 ? g[m] : gs[i][lane] + g[m];
+                    }
+                }
+                __syncthreads();
+            }
+        }
+        for (int p = wave; p < kPoints; p += P) {
+            vr F(0, 0, 0);
+            const double px = rs[3 * p][lane], py = rs[3 * p + 1][lane], pz = rs[3 * p + 2][lane];
+#pragma unroll 2
+            for (int c = 0; c < tab->count[p]; ++c) {
+                const int n = tab->with[p][c].n, o = 3 * tab->with[p][c].other;
+                const vr d((real)(px - rs[o][lane]), (real)(py - rs[o + 1][lane]), (real)(pz - rs[o + 2][lane]));
+                const real ri = rsqrt_pip(d.dot(d)), k = (real)tab->with[p][c].k;
+                const real gg = -(tab->with[p][c].coul ? k + ri : k) * xs[n][lane] * ri;
+                F += d * (gg * gs[n][lane]);
+            }
+            fs[3 * p][lane] = F.x;
+            fs[3 * p + 1][lane] = F.y;
+            fs[3 * p + 2][lane] = F.z;
+        }
+        __syncthreads();
+        if (wave <= kMols) {
+            real E = es[0][lane];
+#pragma unroll
+            for (int w = 1; w < P; ++w) E += es[w][lane];
+            unit_end(wave, on, t, t < nu, (double)E, rs, fs, list, idx, force, energy, eunit, lane);
+        }
+        __syncthreads();  // the LDS arrays are written again
+    }
+}
+#endif
 
 }  // namespace
 }  // namespace mbpol
@@ -519,18 +872,45 @@ __global__ void __launch_bounds__(64) PIP3_OCCUPANCY k_threebody(long long nt, c
 #define PIP_CAT2(a, b) a##b
 #define PIP_CAT(a, b) PIP_CAT2(a, b)
 namespace mbpol {
-// one 64-lane block per 64 units, at most max_blocks (when positive)
-static inline int grid(long long n, int max_blocks) {
-    const long long b = (n + 63) / 64;
-    return (int)(max_blocks > 0 && b > max_blocks ? max_blocks : b);
+// one block of `waves` waves per 64 units, at most max_waves waves (when positive)
+static inline int grid(long long n, int max_waves, int waves) {
+    const long long b = (n + 63) / 64, cap = std::max(1, max_waves / waves);
+    return (int)(max_waves > 0 && b > cap ? cap : b);
 }
+#if PIP_ORBIT
+// Blocks a unit's passes are spread over: as many as still find a CU each, since
+// only then does every wave have a SIMD to itself, and a short list takes as long
+// as one wave's passes.  Not with unit energies, which one block writes whole.
+static int unit_parts(long long n, bool eunit) {
+    static const int cus = [] {
+        int d = 0, c = 0;
+        const bool ok = hipGetDevice(&d) == hipSuccess &&
+                        hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, d) == hipSuccess;
+        return ok && c > 0 ? c : 256;
+    }();
+    const long long units = (n + 63) / 64;
+    for (int q : {6, 3, 2})
+        if (!eunit && kPassAll % (P * q) == 0 && units * q <= cus) return q;
+    return 1;
+}
+#define PIP_LAUNCH(kern, n, s, ...)                                                                         \
+    do {                                                                                                    \
+        const int parts = unit_parts(n, eunit != nullptr);                                                  \
+        MBPOL_LAUNCH(ev, k_pip_split, parts > 1 ? parts * grid(n, 0, P) : grid(n, max_blocks, P), 64 * P, 0, \
+                     s, parts, __VA_ARGS__);                                                                \
+    } while (0)
+#else
+#define PIP_LAUNCH(kern, n, s, ...) MBPOL_LAUNCH(ev, kern, grid(n, max_blocks, 1), 64, 0, s, __VA_ARGS__)
+#endif
 #if PIP_BODY == 2
 void PIP_CAT(launch_twobody_, PIP_SUFFIX)(hipStream_t s, long long npairs, const long long* ndev, const int2* pairs,
                                           const int* idx, const double* pos, int periodic, d3 box, u64* force,
                                           u64* energy, const KEvents& ev, double* eunit, int max_blocks) {
-    const d3 boxA{box.x * 10., box.y * 10., box.z * 10.};
+#if !PIP_ORBIT
+    box = d3{box.x * 10., box.y * 10., box.z * 10.};
+#endif
     if (npairs > 0)
-        MBPOL_LAUNCH(ev, k_twobody, grid(npairs, max_blocks), 64, 0, s, npairs, ndev, pairs, idx, pos, periodic, boxA,
+        PIP_LAUNCH(k_twobody, npairs, s, npairs, ndev, pairs, idx, pos, periodic, box,
                      force, energy, eunit);
 }
 #else
@@ -538,7 +918,7 @@ void PIP_CAT(launch_threebody_, PIP_SUFFIX)(hipStream_t s, long long ntrip, cons
                                             const int* idx, const double* pos, int periodic, d3 box, u64* force,
                                             u64* energy, const KEvents& ev, double* eunit, int max_blocks) {
     if (ntrip > 0)
-        MBPOL_LAUNCH(ev, k_threebody, grid(ntrip, max_blocks), 64, 0, s, ntrip, ndev, trip, idx, pos, periodic, box,
+        PIP_LAUNCH(k_threebody, ntrip, s, ntrip, ndev, trip, idx, pos, periodic, box,
                      force, energy, eunit);
 }
 #endif

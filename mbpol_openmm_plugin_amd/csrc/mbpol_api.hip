@@ -27,11 +27,10 @@ static int pip3_kernel_choice() {
     const char* env = std::getenv("MBPOL_HIP_3B_KERNEL");
     return env && !std::strcmp(env, "terms") ? 1 : 0;
 }
-// the 2-body kernel: term by term unless MBPOL_HIP_2B_KERNEL=orbit (the loop over
-// the dimer's relabelling group, 0.7% slower over a whole evaluation)
+// the 2-body kernel: the same choice (MBPOL_HIP_2B_KERNEL)
 static int pip2_kernel_choice() {
     const char* env = std::getenv("MBPOL_HIP_2B_KERNEL");
-    return env && !std::strcmp(env, "orbit") ? 0 : 1;
+    return env && !std::strcmp(env, "terms") ? 1 : 0;
 }
 
 static thread_local std::string g_last_error;

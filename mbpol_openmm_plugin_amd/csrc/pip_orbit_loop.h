@@ -43,15 +43,16 @@ struct pip_orbit_tables<float> {
     }
 };
 
-// R(x) + the passes of Q over the group; g receives dE/dx (overwritten), x is
-// left as it was.  Pass(x, g, cf) adds one pass's energy gradient into g.
-template <typename T, int N, typename Rest, typename Pass, typename Table>
-__host__ __device__ __forceinline__ T pip_orbit_eval(T (&x)[N], T (&g)[N], Rest rest, Pass pass, Table table,
-                                                     int npass, unsigned step_mask, const int (&step_a)[N],
-                                                     const int (&step_b)[N]) {
-    T e = rest(x, g);
+// Passes k0 .. k1 - 1 of Q over the group.  On entry the registers hold the
+// labelling before pass k0, on return the one after pass k1 - 1.
+// Pass(x, g, cf) adds one pass's gradient into g and returns its energy.
+template <typename T, int N, typename Pass, typename Table>
+__host__ __device__ __forceinline__ T pip_orbit_passes(T (&x)[N], T (&g)[N], Pass pass, Table table, int k0, int k1,
+                                                       unsigned step_mask, const int (&step_a)[N],
+                                                       const int (&step_b)[N]) {
+    T e = T(0);
 #pragma nounroll
-    for (int k = 0; k < npass; ++k) {
+    for (int k = k0; k < k1; ++k) {
         auto cf = table();
         PIP_OPAQUE_PTR(cf);
         e += pass(x, g, cf);
@@ -78,22 +79,31 @@ __host__ __device__ __forceinline__ T pip_orbit_eval(T (&x)[N], T (&g)[N], Rest 
     return e;
 }
 
+template <typename T>
+__host__ __device__ __forceinline__ T pip3b_orbit_passes(T (&x)[36], T (&g)[36], int k0, int k1) {
+    return pip_orbit_passes<T, 36>(
+        x, g, [](T (&y)[36], T (&h)[36], PIP_CONST_PTR(T) cf) { return pip3b_orbit_pass<T>(y, h, cf); },
+        [] { return pip_orbit_tables<T>::trimer(); }, k0, k1, pip3b_step_mask, pip3b_step_a, pip3b_step_b);
+}
+template <typename T>
+__host__ __device__ __forceinline__ T pip2b_orbit_passes(T (&x)[31], T (&g)[31], int k0, int k1) {
+    return pip_orbit_passes<T, 31>(
+        x, g, [](T (&y)[31], T (&h)[31], PIP_CONST_PTR(T) cf) { return pip2b_orbit_pass<T>(y, h, cf); },
+        [] { return pip_orbit_tables<T>::dimer(); }, k0, k1, pip2b_step_mask, pip2b_step_a, pip2b_step_b);
+}
+
 // E(x) and dE/dx (into g, overwritten) of the 3-body polynomial; x is left as it was.
 template <typename T>
 __host__ __device__ __forceinline__ T pip3b_orbit_eval(T (&x)[36], T (&g)[36]) {
-    return pip_orbit_eval<T, 36>(
-        x, g, [](T (&y)[36], T (&h)[36]) { return pip3b_rest<T>(y, h); },
-        [](T (&y)[36], T (&h)[36], PIP_CONST_PTR(T) cf) { return pip3b_orbit_pass<T>(y, h, cf); },
-        [] { return pip_orbit_tables<T>::trimer(); }, pip3b_npass, pip3b_step_mask, pip3b_step_a, pip3b_step_b);
+    const T e = pip3b_rest<T>(x, g);
+    return e + pip3b_orbit_passes<T>(x, g, 0, pip3b_npass);
 }
 
-// the same for the 2-body polynomial
+// the same for the 2-body polynomial (R is empty)
 template <typename T>
 __host__ __device__ __forceinline__ T pip2b_orbit_eval(T (&x)[31], T (&g)[31]) {
-    return pip_orbit_eval<T, 31>(
-        x, g, [](T (&y)[31], T (&h)[31]) { return pip2b_rest<T>(y, h); },
-        [](T (&y)[31], T (&h)[31], PIP_CONST_PTR(T) cf) { return pip2b_orbit_pass<T>(y, h, cf); },
-        [] { return pip_orbit_tables<T>::dimer(); }, pip2b_npass, pip2b_step_mask, pip2b_step_a, pip2b_step_b);
+    const T e = pip2b_rest<T>(x, g);
+    return e + pip2b_orbit_passes<T>(x, g, 0, pip2b_npass);
 }
 
 }  // namespace mbpol
