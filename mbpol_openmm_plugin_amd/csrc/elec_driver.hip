@@ -104,12 +104,8 @@ struct Elec {
     DevBuf phi_fix, phi_ind, fsite, V, eblk;
     // PME
     DevBuf grid, spec, influence, bx, by, bz;
-    BrickGeom B{};
-    struct Bins {
-        DevBuf of, count, start, fill, members;
-    } binq;  // sites with a charge, by grid brick
     DevBuf g0tab, sptab;  // per-site spline table
-    DevBuf rowcount, rowstart, rowfill, esite, ecoef;  // dipole-spreading table in grid-point order
+    DevBuf rowcount, rowstart, rowfill, ecode, esz, ecoef;  // spreading table by grid line
     // grid transforms: the library's own passes (kernels_fft.hip, kernels_dft.hip) when every
     // axis has a form there (fft_plan), else hipFFT
     PmeFft fft{};
@@ -241,12 +237,12 @@ static bool fft_factor(int n, FftAxis& a) {
 // The mixed radix is the better one only where two radices make up the length
 // (16 lanes a line, so that its tiles are 8 complex columns wide) and the dense
 // product has grown: x and y from 100 up.  The dense z passes have no front
-// stage, so they stay ahead up to about 250.  A length with a factor above 13
+// stage; with the spreading fused into the forward one they stay ahead to about 320.  A length with a factor above 13
 // has no mixed-radix form; dense, 61 takes 4.2 us (y), 137 16.5, 211 69, 307 220.
 static bool fft_plan(int n, int d, FftAxis& a) {
     const bool smooth = fft_factor(n, a);
     const bool two = smooth && a.lgP <= 4 && n >= 100;
-    a.dense = n <= kDftMaxLength && !(smooth && (d == 2 ? n > 250 : two));
+    a.dense = n <= kDftMaxLength && !(smooth && (d == 2 ? n > 320 : two));
     // front radix of the dense x and y passes: the fewest matrix products, a point
     // of the front stage counted as two
     a.front = 1;
@@ -260,26 +256,6 @@ static bool fft_plan(int n, int d, FftAxis& a) {
         }
     }
     return smooth || a.dense;
-}
-
-// Brick size along one grid axis for the spreading kernel: every brick at least
-// 4 points wide and none above 12 (the last one takes the remainder).
-static void brick_axis(int K, int& s, int& nb) {
-    if (K <= 12) {
-        s = K;
-        nb = 1;
-        return;
-    }
-    for (int c : {9, 10, 8, 11, 12, 7}) {
-        const int r = K % c;
-        if (r == 0 || r >= 4) {
-            s = c;
-            nb = (K + c - 1) / c;
-            return;
-        }
-    }
-    s = 6;  // remainder merged into the last brick: 6..11 points
-    nb = K / 6;
 }
 
 // polarisable-site index list and its host mirror
@@ -499,16 +475,10 @@ int elec_create(mbpol_context* ctx) {
         if (int e = up(ctx->stream, E->bx, bspline_moduli(grid[0]))) return e;
         if (int e = up(ctx->stream, E->by, bspline_moduli(grid[1]))) return e;
         if (int e = up(ctx->stream, E->bz, bspline_moduli(grid[2]))) return e;
-        for (int d = 0; d < 3; ++d) brick_axis(grid[d], E->B.s[d], E->B.nb[d]);
-        const int nbins = E->B.nb[0] * E->B.nb[1] * E->B.nb[2];
-        HIP_TRY(E->binq.of.ensure(sizeof(int) * std::max(n, 1)));
-        HIP_TRY(E->binq.members.ensure(sizeof(int) * std::max(n, 1)));
-        HIP_TRY(E->binq.count.ensure(sizeof(int) * (nbins + 1)));
-        HIP_TRY(E->binq.start.ensure(sizeof(int) * (nbins + 1)));
-        HIP_TRY(E->binq.fill.ensure(sizeof(int) * (nbins + 1)));
         HIP_TRY(E->g0tab.ensure(sizeof(int) * 3 * std::max(n, 1)));
         HIP_TRY(E->sptab.ensure(sizeof(double) * 30 * std::max(n, 1)));
-        for (DevBuf* b : {&E->rowcount, &E->rowstart, &E->rowfill}) HIP_TRY(b->ensure(sizeof(int) * (nreal + 1)));
+        for (DevBuf* b : {&E->rowcount, &E->rowstart, &E->rowfill})
+            HIP_TRY(b->ensure(sizeof(int) * (2 * (size_t)grid[0] * grid[1] + 1)));
         if (lds) {
             for (int d = 0; d < 3; ++d) {
                 const int m = grid[d];
@@ -669,24 +639,21 @@ static int build_rows(mbpol_context* ctx) {
     launch_prefactors_field(st, E->npol, E->polidx.as<int>(), pos, site_params(E), E->P, rows(E), E->pf.as<double2>(),
                             E->efix.as<double>());
     if (E->P.pme) {
-        const int nbins = E->B.nb[0] * E->B.nb[1] * E->B.nb[2];
         launch_site_spline_table(st, n, pos, E->P, E->g0tab.as<int>(), E->sptab.as<double>());
-        // dipole-spreading table
-        const size_t ngrid = (size_t)E->P.grid.x * E->P.grid.y * E->P.grid.z;
-        const size_t nent = (size_t)E->npol * 125;
-        HIP_TRY(E->esite.ensure(sizeof(int) * std::max<size_t>(nent, 1)));
+        // spreading table
+        const int rows2 = 2 * E->P.grid.x * E->P.grid.y;
+        const size_t nent = (size_t)n * 25;
+        HIP_TRY(E->ecode.ensure(sizeof(int) * std::max<size_t>(nent, 1)));
+        HIP_TRY(E->esz.ensure(sizeof(int2) * std::max<size_t>(nent, 1)));
         HIP_TRY(E->ecoef.ensure(sizeof(double) * 3 * std::max<size_t>(nent, 1)));
-        launch_csr_count(st, E->npol, E->polidx.as<int>(), E->g0tab.as<int>(), E->P, E->rowcount.as<int>());
-        if (int e = scan_i32(ctx, E->rowcount.as<int>(), E->rowstart.as<int>(), (int)ngrid + 1)) return e;
-        launch_csr_fill(st, E->npol, E->polidx.as<int>(), E->g0tab.as<int>(), E->sptab.as<double>(), E->P,
-                        E->rowstart.as<int>(), E->rowfill.as<int>(), E->esite.as<int>(), E->ecoef.as<double>());
-        launch_csr_sort(st, ngrid, E->rowstart.as<int>(), E->esite.as<int>(), E->ecoef.as<double>());
-        // charged sites by brick, for the charge spreading
-        Elec::Bins& b = E->binq;
-        launch_site_bins(st, n, pos, E->q.as<double>(), E->P, E->B, b.of.as<int>(), b.count.as<int>());
-        if (int e = scan_i32(ctx, b.count.as<int>(), b.start.as<int>(), nbins + 1)) return e;
-        launch_bucket_fill(st, n, b.of.as<int>(), b.start.as<int>(), b.fill.as<int>(), E->unsorted.as<int>());
-        launch_rank_sort(st, n, b.of.as<int>(), b.start.as<int>(), E->unsorted.as<int>(), b.members.as<int>());
+        auto table = [&](int stage) {
+            launch_line_table(st, stage, n, E->g0tab.as<int>(), E->sptab.as<double>(), E->pol.as<double>(),
+                              E->q.as<double>(), E->P, E->rowcount.as<int>(), E->rowstart.as<int>(),
+                              E->rowfill.as<int>(), E->ecode.as<int>(), E->esz.as<int2>(), E->ecoef.as<double>());
+        };
+        table(0);
+        if (int e = scan_i32(ctx, E->rowcount.as<int>(), E->rowstart.as<int>(), rows2 + 1)) return e;
+        table(1);
     }
     return MBPOL_OK;
 }
@@ -697,20 +664,19 @@ static int pme_grid(mbpol_context* ctx, int mode, const double* mu, const int* s
     hipStream_t st = ctx->stream;
     const ElecParams& P = E->P;
     const size_t nhalf = (size_t)P.grid.x * P.grid.y * (P.grid.z / 2 + 1);
-    // dipoles through the single-axis LDS passes: spreading and z pass in one kernel
-    const bool fused = mode == 1 && E->lds_fft && !E->plane_fft && E->fuse_spread;
-    if (mode == 0) {
-        launch_spread_bricks(st, mode, E->q.as<double>(), mu, P, E->B, E->binq.start.as<int>(),
-                             E->binq.members.as<int>(), E->g0tab.as<int>(), E->sptab.as<double>(), E->grid.as<double>());
-    } else if (fused) {
-        const KEvents ev = timer_kernel(ctx, T_SPREAD_FFT_Z);
-        launch_spread_fft_z_r2c(st, E->fft, E->rowstart.as<int>(), E->esite.as<int>(), E->ecoef.as<double>(), mu,
-                                E->spec.as<double2>(), ev, stop);
-        timer_kernel_done(ctx, T_SPREAD_FFT_Z, ev);
+    const LineTable T{P.grid.x * P.grid.y, P.grid.z, E->rowstart.as<int>(), E->esz.as<int2>(), E->ecoef.as<double>(),
+                      E->sptab.as<double>(), P.grid.z * P.inv_box.z};
+    // the spreading and a dense z pass of the single-axis passes in one kernel
+    const bool fused = E->lds_fft && !E->plane_fft && E->fuse_spread && E->fft.ax[2].dense;
+    if (fused) {
+        const int cat = mode == 0 ? T_FFT_Z_R2C : T_SPREAD_FFT_Z;
+        const KEvents ev = timer_kernel(ctx, cat);
+        launch_spread_dft_z_r2c(st, E->fft, T, mode == 0, mode == 0 ? E->q.as<double>() : mu, E->spec.as<double2>(), ev,
+                                stop);
+        timer_kernel_done(ctx, cat, ev);
     } else {
-        const KEvents ev = timer_kernel(ctx, T_PME_SPREAD);
-        launch_spread_csr(st, (size_t)P.grid.x * P.grid.y * P.grid.z, E->rowstart.as<int>(), E->esite.as<int>(),
-                          E->ecoef.as<double>(), mu, E->grid.as<double>(), ev, stop);
+        const KEvents ev = mode == 0 ? KEvents() : timer_kernel(ctx, T_PME_SPREAD);
+        launch_spread_lines(st, T, mode == 0, mode == 0 ? E->q.as<double>() : mu, E->grid.as<double>(), ev, stop);
         timer_kernel_done(ctx, T_PME_SPREAD, ev);
     }
     if (E->lds_fft) {
@@ -1068,12 +1034,9 @@ int elec_evaluate(mbpol_context* ctx, u64* energy, const std::function<int()>& a
         L.add(E->maxcnt.p, sizeof(int) * 4);
         L.add(E->efix.p, sizeof(double) * 3 * n);
         if (P.pme) {
-            const size_t ngrid = (size_t)P.grid.x * P.grid.y * P.grid.z;
-            const int nbins = E->B.nb[0] * E->B.nb[1] * E->B.nb[2];
-            L.add(E->rowcount.p, sizeof(int) * (ngrid + 1));
-            L.add(E->rowfill.p, sizeof(int) * (ngrid + 1));
-            L.add(E->binq.count.p, sizeof(int) * (nbins + 1));
-            L.add(E->binq.fill.p, sizeof(int) * (nbins + 1));
+            const size_t rows2 = 2 * (size_t)P.grid.x * P.grid.y;
+            L.add(E->rowcount.p, sizeof(int) * (rows2 + 1));
+            L.add(E->rowfill.p, sizeof(int) * (rows2 + 1));
         }
         L.add(E->ctl.p, sizeof(SolveCtl));
         L.add(E->fsite.p, sizeof(double) * 3 * n);

@@ -45,13 +45,6 @@ struct SolveCtl {
     double eps;      // the reference's measure at the last test
 };
 
-// PME grid bricks: s[d] points per brick along axis d (every brick, the last
-// one included, at least 4 points wide), nb[d] bricks
-struct BrickGeom {
-    int s[3];
-    int nb[3];
-};
-
 void launch_site_charges_copy(hipStream_t s, int n, const double* q0, double* q);
 // dst = src (n doubles) when ctl records a converged stop, else nothing
 void launch_copy_if_converged(hipStream_t s, long long n, const SolveCtl* ctl, const double* src, double* dst);
@@ -71,18 +64,12 @@ void launch_site_lists(hipStream_t s, int lanes, int n, const double* pos, const
 // prefactors of the P rows (into pf) and the real-space fixed field added to field, in one pass
 void launch_prefactors_field(hipStream_t s, int npol, const int* polidx, const double* pos, SiteParams S, ElecParams P,
                              const ElecRows& R, double2* pf, double* field);
-void launch_site_bins(hipStream_t s, int n, const double* pos, const double* weight, ElecParams P, BrickGeom B,
-                      int* bin_of, int* bin_count);
 void launch_site_spline_table(hipStream_t s, int n, const double* pos, ElecParams P, int* g0tab, double* sptab);
-void launch_spread_bricks(hipStream_t s, int mode, const double* q, const double* mu, ElecParams P, BrickGeom B,
-                          const int* bin_start, const int* members, const int* g0tab, const double* sptab,
-                          double* grid);
-void launch_csr_count(hipStream_t s, int npol, const int* polidx, const int* g0tab, ElecParams P, int* rowcount);
-void launch_csr_fill(hipStream_t s, int npol, const int* polidx, const int* g0tab, const double* sptab, ElecParams P,
-                     const int* rowstart, int* fill, int* esite, double* ecoef);
-void launch_csr_sort(hipStream_t s, size_t ngrid, const int* rowstart, int* esite, double* ecoef);
-void launch_spread_csr(hipStream_t s, size_t ngrid, const int* rowstart, const int* esite, const double* ecoef,
-                       const double* mu, double* grid, const KEvents& ev, const int* stop = nullptr);
+// spreading table by grid line (2 grid.x grid.y rows): stage 0 counts the rows' entries, stage 1 (after a scan
+// of the counts into rowstart) fills them; rowcount and rowfill start at zero
+void launch_line_table(hipStream_t s, int stage, int n, const int* g0tab, const double* sptab, const double* pol,
+                       const double* q, ElecParams P, int* rowcount, const int* rowstart, int* rowfill, int* code,
+                       int2* sz, double* coef);
 void launch_convolve(hipStream_t s, size_t nhalf, const double* influence, double2* spec);
 // influence function on the half grid, rows of khp entries (entries kz >= K3/2 + 1 are zero)
 void launch_influence(hipStream_t s, ElecParams P, int khp, const double* bx, const double* by, const double* bz,

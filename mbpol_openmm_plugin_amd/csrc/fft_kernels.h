@@ -34,11 +34,21 @@ constexpr int kFftMaxLength = 1024;
 // stop: when non-null and *stop != 0 at launch, the pass does nothing (a dipole solve that has converged)
 void launch_fft_z_r2c(hipStream_t s, const PmeFft& F, const double* real, double2* H, const KEvents& ev,
                       const int* stop = nullptr);
-// the dipole spreading (rows of the spreading table in grid-point order: rowstart, esite,
-// ecoef; dipoles mu) fused with the z pass: the half spectrum of the dipole grid
-void launch_spread_fft_z_r2c(hipStream_t s, const PmeFft& F, const int* rowstart, const int* esite,
-                             const double* ecoef, const double* mu, double2* H, const KEvents& ev,
-                             const int* stop = nullptr);
+// The spreading table by grid line (kernels_elec.hip): rows 0 .. nlines - 1 the polarisable sites of a line,
+// rows nlines .. 2 nlines - 1 its other charged sites
+struct LineTable {
+    int nlines, nz;  // lines (x, y), points of a line
+    const int* start;
+    const int2* sz;      // site, first z
+    const double* coef;  // 3 per entry
+    const double* sptab; // z splines: sptab[30 site + 20 ..]
+    double scale_z;      // K_z / L_z
+};
+// spreads charges (w = q) or dipoles (w = mu) onto the real grid, or straight into the forward z pass (dense z only)
+void launch_spread_lines(hipStream_t s, const LineTable& T, bool charges, const double* w, double* real,
+                         const KEvents& ev, const int* stop = nullptr);
+void launch_spread_dft_z_r2c(hipStream_t s, const PmeFft& F, const LineTable& T, bool charges, const double* w,
+                             double2* H, const KEvents& ev, const int* stop = nullptr);
 void launch_fft_y(hipStream_t s, const PmeFft& F, double2* H, int inverse, const KEvents& ev,
                   const int* stop = nullptr);
 void launch_fft_x_conv(hipStream_t s, const PmeFft& F, double2* H, const double* influence, const KEvents& ev,
@@ -49,8 +59,6 @@ void launch_fft_z_c2r(hipStream_t s, const PmeFft& F, const double2* H, double* 
 constexpr int kDftMaxLength = 512;
 void launch_dft_z_r2c(hipStream_t s, const PmeFft& F, const double* real, double2* H, const KEvents& ev,
                       const int* stop);
-void launch_spread_dft_z_r2c(hipStream_t s, const PmeFft& F, const int* rowstart, const int* esite,
-                             const double* ecoef, const double* mu, double2* H, const KEvents& ev, const int* stop);
 void launch_dft_y(hipStream_t s, const PmeFft& F, double2* H, int inverse, const KEvents& ev, const int* stop);
 void launch_dft_x_conv(hipStream_t s, const PmeFft& F, double2* H, const double* influence, const KEvents& ev,
                        const int* stop);
