@@ -76,7 +76,7 @@ struct Elec {
     DevBuf cpos;  // positions and polarisable flags in cell order
     int3 nc{1, 1, 1};
     int reach = 1, use_cells = 0;
-    int site_lanes = 0;  // lanes per site of the row build: 0 until tuned on the first evaluation
+    int site_lanes = 0;  // lanes per site of the row build: 0 before the first evaluation
     // neighbour rows (ELL) and induced-field prefactors
     DevBuf nbP, cntP, nbQ, cntQ, pf, maxcnt;
     int capP = 0, capQ = 0;
@@ -518,53 +518,6 @@ static ElecRows rows(const Elec* E) {
                     E->pf.as<double2>()};
 }
 
-// neighbour rows of every site (PME: within the cutoff; direct sum: every
-// other site), the induced-field prefactors, and the PME bins
-// Autotuning of the row build: the lane count per site (8, 16, 32) is timed on
-// this context's own first configuration, each candidate twice (the second
-// launch counts), and the fastest is kept.  Every candidate writes the same
-// rows.  MBPOL_HIP_SITE_LANES=8|16|32 fixes the choice instead.
-static int tune_site_lists(mbpol_context* ctx) {
-    Elec* E = ctx->elec;
-    if (const char* env = std::getenv("MBPOL_HIP_SITE_LANES")) {
-        const int v = std::atoi(env);
-        E->site_lanes = (v == 8 || v == 32) ? v : 16;
-        return MBPOL_OK;
-    }
-    if (!E->use_cells) {  // direct sum: rows of every site, no search to tune
-        E->site_lanes = 16;
-        return MBPOL_OK;
-    }
-    hipStream_t st = ctx->stream;
-    hipEvent_t a = nullptr, b = nullptr;
-    HIP_TRY(hipEventCreate(&a));
-    HIP_TRY(hipEventCreate(&b));
-    float best = 1e30f;
-    int choice = 16;
-    for (int lanes : {8, 16, 32}) {
-        float ms = 0.f;
-        for (int rep = 0; rep < 2; ++rep) {
-            launch_fill_zero(st, E->maxcnt.p, sizeof(int) * 4);
-            HIP_TRY(hipEventRecord(a, st));
-            launch_site_lists(st, lanes, E->n, ctx->pos.as<double>(), E->pol.as<double>(), E->P, E->nc, E->reach,
-                              E->use_cells, E->cell_of.as<int>(), E->cell_start.as<int>(), E->members.as<int>(),
-                              E->cpos.as<double4>(), E->capP, E->capQ, E->nbP.as<int>(), E->cntP.as<int>(),
-                              E->nbQ.as<int>(), E->cntQ.as<int>(), E->maxcnt.as<int>());
-            HIP_TRY(hipEventRecord(b, st));
-            HIP_TRY(hipEventSynchronize(b));
-            HIP_TRY(hipEventElapsedTime(&ms, a, b));
-        }
-        if (ms < best) {
-            best = ms;
-            choice = lanes;
-        }
-    }
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
-    E->site_lanes = choice;
-    return MBPOL_OK;
-}
-
 int elec_tuning(const mbpol_context* ctx, const char* name, int* value) {
     const Elec* E = ctx->elec;
     if (E && std::strcmp(name, "site_lanes") == 0)
@@ -594,41 +547,35 @@ static int build_rows(mbpol_context* ctx) {
         launch_site_pack(st, n, E->members.as<int>(), pos, E->pol.as<double>(), E->cpos.as<double4>());
     }
     int* h = reinterpret_cast<int*>(E->h_eps) + 8;
+    auto build = [&]() -> int {
+        const size_t rp = (size_t)n * E->capP, rq = (size_t)n * E->capQ;
+        HIP_TRY(E->nbP.ensure(sizeof(int) * std::max<size_t>(rp, 1)));
+        HIP_TRY(E->pf.ensure(sizeof(double2) * std::max<size_t>(rp, 1)));
+        HIP_TRY(E->nbQ.ensure(sizeof(int) * std::max<size_t>(rq, 1)));
+        launch_site_lists(st, n, pos, E->pol.as<double>(), E->P, E->nc, E->reach, E->use_cells, E->cell_of.as<int>(),
+                          E->cell_start.as<int>(), E->cpos.as<double4>(), E->capP, E->capQ, E->nbP.as<int>(),
+                          E->cntP.as<int>(), E->nbQ.as<int>(), E->cntQ.as<int>(), E->maxcnt.as<int>());
+        HIP_TRY(hipMemcpyAsync(h, E->maxcnt.p, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
+        return MBPOL_OK;
+    };
     E->rows_pending = false;
     if (!E->rows_sync && E->site_lanes > 0) {
         // The rows' maxima reach the host with the energies; elec_rows_check
         // compares them with the capacities after the evaluation and has it
         // redone when a row overflowed (the kernels clamp to the capacity, so an
         // overflowing row loses neighbours but nothing is written out of bounds).
-        const size_t rp = (size_t)n * E->capP, rq = (size_t)n * E->capQ;
-        HIP_TRY(E->nbP.ensure(sizeof(int) * std::max<size_t>(rp, 1)));
-        HIP_TRY(E->pf.ensure(sizeof(double2) * std::max<size_t>(rp, 1)));
-        HIP_TRY(E->nbQ.ensure(sizeof(int) * std::max<size_t>(rq, 1)));
-        launch_site_lists(st, E->site_lanes, n, pos, E->pol.as<double>(), E->P, E->nc, E->reach, E->use_cells,
-                          E->cell_of.as<int>(), E->cell_start.as<int>(), E->members.as<int>(), E->cpos.as<double4>(),
-                          E->capP, E->capQ, E->nbP.as<int>(), E->cntP.as<int>(), E->nbQ.as<int>(), E->cntQ.as<int>(),
-                          E->maxcnt.as<int>());
-        HIP_TRY(hipMemcpyAsync(h, E->maxcnt.p, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
+        if (int e = build()) return e;
         E->rows_pending = true;
     } else for (int attempt = 0; attempt < 2; ++attempt) {
-        const size_t rp = (size_t)n * E->capP, rq = (size_t)n * E->capQ;
-        HIP_TRY(E->nbP.ensure(sizeof(int) * std::max<size_t>(rp, 1)));
-        HIP_TRY(E->pf.ensure(sizeof(double2) * std::max<size_t>(rp, 1)));
-        HIP_TRY(E->nbQ.ensure(sizeof(int) * std::max<size_t>(rq, 1)));
         launch_fill_zero(st, E->maxcnt.p, sizeof(int) * 4);
-        launch_site_lists(st, E->site_lanes > 0 ? E->site_lanes : 16, n, pos, E->pol.as<double>(), E->P, E->nc, E->reach,
-                          E->use_cells, E->cell_of.as<int>(), E->cell_start.as<int>(), E->members.as<int>(),
-                          E->cpos.as<double4>(), E->capP, E->capQ, E->nbP.as<int>(), E->cntP.as<int>(),
-                          E->nbQ.as<int>(), E->cntQ.as<int>(), E->maxcnt.as<int>());
-        HIP_TRY(hipMemcpyAsync(h, E->maxcnt.p, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
+        if (int e = build()) return e;
         HIP_TRY(hipStreamSynchronize(st));
         if (h[0] <= E->capP && h[1] <= E->capQ) break;
         if (attempt == 1) return set_error(MBPOL_ERR_HIP, "electrostatics neighbour rows overflowed twice");
         E->capP = std::max(E->capP, (h[0] + h[0] / 4 + 63) / 32 * 32);
         E->capQ = std::max(E->capQ, (h[1] + h[1] / 4 + 63) / 32 * 32);
     }
-    if (E->site_lanes == 0)
-        if (int e = tune_site_lists(ctx)) return e;
+    E->site_lanes = E->use_cells ? 64 : 16;
     if (!E->rows_pending) {
         E->rows_sync = false;
         ctx->stats.elec_pairs = h[2] / 2;

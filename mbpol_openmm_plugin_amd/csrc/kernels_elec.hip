@@ -214,125 +214,217 @@ __global__ void k_rank_sort(int n, const int* __restrict__ bucket_of, const int*
 
 // Neighbour rows of every site, in fixed-capacity (ELL) layout: row i of the
 // P table lists the polarisable sites j != i with r_ij <= rc (minimum image
-// under PME), row i of the Q table the non-polarisable ones.  One group of G
-// lanes per site; candidates are taken in cell order and compacted with a
-// wavefront ballot.  Counts are kept beyond the capacity so that the host can
-// detect an overflow (maxcnt[0..1]) and rebuild with larger rows; maxcnt[2]
-// accumulates the number of directed pairs, maxcnt[3] the P entries of the
-// polarisable sites (the rows the dipole iteration streams).
-// positions and polarisable flags in cell order: the row build reads its
-// candidates from consecutive entries instead of gathering them by site index
+// under PME), row i of the Q table the non-polarisable ones.  Candidates are taken
+// in cell order and compacted with a wavefront ballot.  Counts are kept beyond the
+// capacity so that the host can detect an overflow (maxcnt[0..1]) and rebuild with
+// larger rows; maxcnt[2] accumulates the number of directed pairs, maxcnt[3] the P
+// entries of the polarisable sites (the rows the dipole iteration streams).
+struct RowBuild {
+    int capP, capQ;
+    int *nbP, *cntP, *nbQ, *cntQ, *maxcnt;
+};
+
+// The G lanes of a group append what they found near site i: q holds the position of j and 2 j + (j is polarisable)
+template <int G>
+__device__ __forceinline__ void row_consider(int i, double xi, double yi, double zi, double rc2, const ElecParams& P,
+                                             const RowBuild& B, bool active, const double4& q, int& cP, int& cQ) {
+    const unsigned long long gb = group_bits<G>(), below = lanes_below();
+    const int code = (int)q.w, j = code >> 1;
+    bool ok = false;
+    if (active && j != i) {
+        double dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
+        min_image(dx, dy, dz, P);
+        ok = dx * dx + dy * dy + dz * dz <= rc2;
+    }
+    const bool inP = ok && (code & 1), inQ = ok && !(code & 1);
+    const unsigned long long bP = __ballot(inP) & gb, bQ = __ballot(inQ) & gb;
+    if (inP) {
+        const int k = cP + __popcll(bP & below);
+        if (k < B.capP) B.nbP[(size_t)i * B.capP + k] = j;
+    }
+    if (inQ) {
+        const int k = cQ + __popcll(bQ & below);
+        if (k < B.capQ) B.nbQ[(size_t)i * B.capQ + k] = j;
+    }
+    cP += __popcll(bP);
+    cQ += __popcll(bQ);
+}
+
+// row maxima and totals: combined in LDS, one set of global atomics per block
+struct RowTotals {
+    int v[4];
+};
+__device__ __forceinline__ void row_totals_add(RowTotals& red, int cP, int cQ, bool polarisable) {
+    atomicMax(&red.v[0], cP);
+    atomicMax(&red.v[1], cQ);
+    atomicAdd(&red.v[2], cP + cQ);
+    if (polarisable) atomicAdd(&red.v[3], cP);
+}
+__device__ __forceinline__ void row_totals_out(const RowTotals& red, int* __restrict__ maxcnt) {
+    if (threadIdx.x == 0) {
+        atomicMax(&maxcnt[0], red.v[0]);
+        atomicMax(&maxcnt[1], red.v[1]);
+        atomicAdd(&maxcnt[2], red.v[2]);
+        atomicAdd(&maxcnt[3], red.v[3]);
+    }
+}
+
+// without cells: every site (of the group) is a candidate, G lanes per site
+template <int G>
+__global__ void __launch_bounds__(256) k_site_lists(int n, const double* __restrict__ pos, const double* __restrict__ pol,
+                                                    ElecParams P, RowBuild B) {
+    critical_path_wave();
+    const int i = (blockIdx.x * blockDim.x + threadIdx.x) / G, lane = threadIdx.x % G;
+    __shared__ RowTotals red;
+    if (threadIdx.x < 4) red.v[threadIdx.x] = 0;
+    __syncthreads();
+    if (i < n) {  // uniform over the group
+        const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2], rc2 = P.cutoff * P.cutoff;
+        int cP = 0, cQ = 0;
+        const int b0 = P.gs ? P.gs[i] : 0, b1 = P.gs ? P.ge[i] : n;
+        for (int b = b0; b < b1; b += G) {
+            const int j = b + lane;
+            const bool act = j < b1;
+            row_consider<G>(i, xi, yi, zi, rc2, P, B, act,
+                            act ? make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2],
+                                               2.0 * j + (pol[j] != 0.0 ? 1.0 : 0.0))
+                                : make_double4(0.0, 0.0, 0.0, 0.0),
+                            cP, cQ);
+        }
+        if (lane == 0) {
+            B.cntP[i] = cP;
+            B.cntQ[i] = cQ;
+            row_totals_add(red, cP, cQ, pol[i] != 0.0);
+        }
+    }
+    __syncthreads();
+    row_totals_out(red, B.maxcnt);
+}
+
+// positions in cell order with 2 j + (site j is polarisable): the row build reads
+// its candidates from consecutive entries
 __global__ void k_site_pack(int n, const int* __restrict__ members, const double* __restrict__ pos,
                             const double* __restrict__ pol, double4* __restrict__ cpos) {
     critical_path_wave();
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const int j = members[t];
-    cpos[t] = make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], pol[j] != 0.0 ? 1.0 : 0.0);
+    cpos[t] = make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], 2.0 * j + (pol[j] != 0.0 ? 1.0 : 0.0));
 }
 
-template <int G>
-__global__ void __launch_bounds__(256) k_site_lists(int n, const double* __restrict__ pos, const double* __restrict__ pol,
-                                                    ElecParams P, int3 nc, int reach, int use_cells,
-                                                    const int* __restrict__ cell_of, const int* __restrict__ cell_start,
-                                                    const int* __restrict__ members,
-                                                    const double4* __restrict__ cpos, int capP, int capQ,
-                                                    int* __restrict__ nbP, int* __restrict__ cntP,
-                                                    int* __restrict__ nbQ, int* __restrict__ cntQ,
-                                                    int* __restrict__ maxcnt) {
+// With cells: a wave takes kRowSites consecutive sites of the cell order and tests
+// every candidate it loads against those of them that share the cell.  The cells
+// (X, Y, Z - reach .. Z + reach) are consecutive in the cell order, so a column is
+// one or two member ranges (about 60 members at reach 2); all ranges are found at
+// once, one per lane, laid end to end and walked 64 members at a time, the next ones
+// loaded ahead.
+// What bounds it: the traffic of the candidates (1500 entries of 32 bytes a site)
+// with one site a wave -- 220 us for 16,384 sites, 127 us for 8788; with 16 or 32
+// lanes a site walking range after range, latency, 127 us for both; now 93 and 74 us, bound
+// by the instructions of the tests (about 45 for 64 candidates and a site).
+constexpr int kRowSites = 4;
+__global__ void __launch_bounds__(256) k_site_lists_cells(int n, ElecParams P, int3 nc, int reach,
+                                                          const int* __restrict__ cell_of,
+                                                          const int* __restrict__ cell_start,
+                                                          const double4* __restrict__ cpos, RowBuild B) {
     critical_path_wave();
-    const int i = (blockIdx.x * blockDim.x + threadIdx.x) / G, lane = threadIdx.x % G;
-    int cP = 0, cQ = 0;
-    if (i < n) {  // uniform over the group
-    const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
+    __shared__ RowTotals red;
+    if (threadIdx.x < 4) red.v[threadIdx.x] = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int t0 = kRowSites * __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const int ns = min(kRowSites, n - t0);  // <= 0: no sites left
     const double rc2 = P.cutoff * P.cutoff;
-    const unsigned long long gb = group_bits<G>(), below = lanes_below();
-    int* rowP = nbP + (size_t)i * capP;
-    int* rowQ = nbQ + (size_t)i * capQ;
-    // q: position of j and 1 if j is polarisable (from the cell-ordered copy when cells are used)
-    auto consider = [&](int j, bool active, const double4& q) {
-        bool ok = false, pj = false;
-        if (active && j != i) {
-            double dx = q.x - xi, dy = q.y - yi, dz = q.z - zi;
-            min_image(dx, dy, dz, P);
-            ok = dx * dx + dy * dy + dz * dz <= rc2;
-            pj = q.w != 0.0;
+    int cP[kRowSites], cQ[kRowSites], code[kRowSites], cell[kRowSites];
+    double4 at[kRowSites];
+#pragma unroll
+    for (int u = 0; u < kRowSites; ++u) {
+        cP[u] = cQ[u] = 0;
+        at[u] = u < ns ? cpos[t0 + u] : make_double4(0.0, 0.0, 0.0, 0.0);
+        code[u] = __builtin_amdgcn_readfirstlane((int)at[u].w);
+        cell[u] = u < ns ? __builtin_amdgcn_readfirstlane(cell_of[code[u] >> 1]) : -1;
+    }
+    for (int first = 0; first < ns;) {
+        int last = first, c = -1;  // the sites first .. last - 1 share cell c
+#pragma unroll
+        for (int u = 0; u < kRowSites; ++u) {
+            if (u == first) c = cell[u];
+            if (u == last && u < ns && cell[u] == c) ++last;
         }
-        const bool inP = ok && pj, inQ = ok && !pj;
-        const unsigned long long bP = __ballot(inP) & gb, bQ = __ballot(inQ) & gb;
-        if (inP) {
-            const int k = cP + __popcll(bP & below);
-            if (k < capP) rowP[k] = j;
-        }
-        if (inQ) {
-            const int k = cQ + __popcll(bQ & below);
-            if (k < capQ) rowQ[k] = j;
-        }
-        cP += __popcll(bP);
-        cQ += __popcll(bQ);
-    };
-    if (!use_cells) {
-        const int b0 = P.gs ? P.gs[i] : 0, b1 = P.gs ? P.ge[i] : n;
-        for (int b = b0; b < b1; b += G) {
-            const int j = b + lane;
-            const bool act = j < b1;
-            const double4 q = act ? make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], pol[j] != 0.0 ? 1.0 : 0.0)
-                                  : make_double4(0.0, 0.0, 0.0, 0.0);
-            consider(j, act, q);
-        }
-    } else {
-        // cells (X, Y, Z - reach .. Z + reach) are consecutive in the cell order, so each
-        // (X, Y) column is one or two contiguous member ranges, visited in the same order
-        // as cell by cell
-        const int cell = cell_of[i];
-        const int cz = cell % nc.z, cy = (cell / nc.z) % nc.y, cx = cell / (nc.z * nc.y);
-        auto scan = [&](int base, int za, int zb) {
-            const int b0 = cell_start[base + za], b1 = cell_start[base + zb + 1];
-            for (int t = b0; t < b1; t += G) {
-                const int tt = t + lane;
-                const bool act = tt < b1;
-                consider(act ? members[tt] : -1, act, act ? cpos[tt] : make_double4(0.0, 0.0, 0.0, 0.0));
+        // range of lane l: column l / 2 (in the order of X, then Y), its first (l even) or second part
+        const int side = 2 * reach + 1;
+        int b = 0, e = 0;
+        if (lane < 2 * side * side) {
+            const int cz = c % nc.z, cy = (c / nc.z) % nc.y, cx = c / (nc.z * nc.y);
+            const int col = lane >> 1;
+            int X = cx + col / side - reach, Y = cy + col % side - reach;
+            X = X < 0 ? X + nc.x : (X >= nc.x ? X - nc.x : X);
+            Y = Y < 0 ? Y + nc.y : (Y >= nc.y ? Y - nc.y : Y);
+            const int z0 = cz - reach, z1 = cz + reach;
+            int za, zb;
+            if (lane & 1) {  // what lies beyond the boundary, when the column crosses it
+                za = 0;
+                zb = z0 < 0 ? z1 : (z1 >= nc.z ? z1 - nc.z : -1);
+            } else {
+                za = z0 < 0 ? z0 + nc.z : z0;
+                zb = z0 < 0 ? nc.z - 1 : min(z1, nc.z - 1);
             }
-        };
-        for (int ax = -reach; ax <= reach; ++ax)
-            for (int ay = -reach; ay <= reach; ++ay) {
-                int X = cx + ax, Y = cy + ay;
-                X = X < 0 ? X + nc.x : (X >= nc.x ? X - nc.x : X);
-                Y = Y < 0 ? Y + nc.y : (Y >= nc.y ? Y - nc.y : Y);
-                const int base = (X * nc.y + Y) * nc.z, z0 = cz - reach, z1 = cz + reach;
-                if (z0 < 0) {
-                    scan(base, z0 + nc.z, nc.z - 1);
-                    scan(base, 0, z1);
-                } else if (z1 >= nc.z) {
-                    scan(base, z0, nc.z - 1);
-                    scan(base, 0, z1 - nc.z);
-                } else {
-                    scan(base, z0, z1);
+            if (za <= zb) {
+                const int base = (X * nc.y + Y) * nc.z;
+                b = cell_start[base + za];
+                e = cell_start[base + zb + 1];
+            }
+        }
+        unsigned long long left = __ballot(e > b);
+        int rb = 0, re = 0;
+        // the next 64 members, over as many ranges as they take
+        auto load = [&](double4& q, bool& act) -> bool {
+            int filled = 0, from = -1;
+            while (filled < 64) {
+                if (rb >= re) {
+                    if (!left) break;
+                    const int r = __builtin_ctzll(left);
+                    left &= left - 1;
+                    rb = __builtin_amdgcn_readlane(b, r);
+                    re = __builtin_amdgcn_readlane(e, r);
                 }
+                const int take = min(64 - filled, re - rb);
+                if (lane >= filled && lane < filled + take) from = rb + lane - filled;
+                rb += take;
+                filled += take;
             }
+            act = from >= 0;
+            if (act) q = cpos[from];
+            return filled > 0;
+        };
+        auto test = [&](bool act, const double4& q) {
+#pragma unroll
+            for (int u = 0; u < kRowSites; ++u)
+                if (first <= u && u < last)
+                    row_consider<64>(code[u] >> 1, at[u].x, at[u].y, at[u].z, rc2, P, B, act, q, cP[u], cQ[u]);
+        };
+        double4 q0 = make_double4(0.0, 0.0, 0.0, 0.0), q1 = q0;
+        bool a0 = false, a1 = false;
+        bool have = load(q0, a0);
+        while (have) {
+            const bool more = load(q1, a1);
+            test(a0, q0);
+            if (!more) break;
+            have = load(q0, a0);
+            test(a1, q1);
+        }
+        first = last;
     }
-    if (lane == 0) {
-        cntP[i] = cP;
-        cntQ[i] = cQ;
-    }
-    }
-    // row maxima and totals: combined in LDS, one set of global atomics per block
-    __shared__ int red[4];
-    if (threadIdx.x < 4) red[threadIdx.x] = 0;
+    if (lane == 0)
+#pragma unroll
+        for (int u = 0; u < kRowSites; ++u)
+            if (u < ns) {
+                B.cntP[code[u] >> 1] = cP[u];
+                B.cntQ[code[u] >> 1] = cQ[u];
+                row_totals_add(red, cP[u], cQ[u], code[u] & 1);
+            }
     __syncthreads();
-    if (i < n && lane == 0) {
-        atomicMax(&red[0], cP);
-        atomicMax(&red[1], cQ);
-        atomicAdd(&red[2], cP + cQ);
-        if (pol[i] != 0.0) atomicAdd(&red[3], cP);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        atomicMax(&maxcnt[0], red[0]);
-        atomicMax(&maxcnt[1], red[1]);
-        atomicAdd(&maxcnt[2], red[2]);
-        atomicAdd(&maxcnt[3], red[3]);
-    }
+    row_totals_out(red, B.maxcnt);
 }
 
 // visit every neighbour of site i (P row, then Q row) with G lanes
@@ -1482,19 +1574,15 @@ void launch_rank_sort(hipStream_t s, int n, const int* bucket_of, const int* buc
 void launch_site_pack(hipStream_t s, int n, const int* members, const double* pos, const double* pol, double4* cpos) {
     if (n > 0) hipLaunchKernelGGL(k_site_pack, nblk(n, 256), 256, 0, s, n, members, pos, pol, cpos);
 }
-void launch_site_lists(hipStream_t s, int lanes, int n, const double* pos, const double* pol, ElecParams P, int3 nc,
-                       int reach, int use_cells, const int* cell_of, const int* cell_start, const int* members,
-                       const double4* cpos, int capP, int capQ, int* nbP, int* cntP, int* nbQ, int* cntQ,
-                       int* maxcnt) {
-#define MBPOL_SITE_LISTS(G)                                                                                          \
-    hipLaunchKernelGGL(k_site_lists<G>, nblk((long long)n * G, 256), 256, 0, s, n, pos, pol, P, nc, reach, use_cells, \
-                       cell_of, cell_start, members, cpos, capP, capQ, nbP, cntP, nbQ, cntQ, maxcnt)
-    switch (lanes) {
-        case 8: MBPOL_SITE_LISTS(8); break;
-        case 32: MBPOL_SITE_LISTS(32); break;
-        default: MBPOL_SITE_LISTS(16); break;
-    }
-#undef MBPOL_SITE_LISTS
+void launch_site_lists(hipStream_t s, int n, const double* pos, const double* pol, ElecParams P, int3 nc,
+                       int reach, int use_cells, const int* cell_of, const int* cell_start, const double4* cpos,
+                       int capP, int capQ, int* nbP, int* cntP, int* nbQ, int* cntQ, int* maxcnt) {
+    const RowBuild B{capP, capQ, nbP, cntP, nbQ, cntQ, maxcnt};
+    if (use_cells)
+        hipLaunchKernelGGL(k_site_lists_cells, nblk(nblk(n, kRowSites) * 64LL, 256), 256, 0, s, n, P, nc, reach, cell_of,
+                           cell_start, cpos, B);
+    else
+        hipLaunchKernelGGL(k_site_lists<kG>, nblk((long long)n * kG, 256), 256, 0, s, n, pos, pol, P, B);
 }
 void launch_prefactors_field(hipStream_t s, int npol, const int* polidx, const double* pos, SiteParams S, ElecParams P,
                              const ElecRows& R, double2* pf, double* field) {
