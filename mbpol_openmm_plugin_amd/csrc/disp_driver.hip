@@ -40,11 +40,14 @@ int disp_set_box(mbpol_context* ctx) {
     D->g.periodic = s.ds_method == MBPOL_CUTOFF_PERIODIC;
     D->g.use_cells = 0;
     D->g.nc = make_int3(1, 1, 1);
-    if (D->g.periodic) {
+    // cells of half the cutoff searched two each way, else of the cutoff searched one each way, else none
+    for (int reach = 2; D->g.periodic && reach >= 1 && !D->g.use_cells; --reach) {
         int nc[3];
-        for (int d = 0; d < 3; ++d) nc[d] = (int)std::floor(s.box[d] / s.ds_cutoff);
-        if (nc[0] >= 3 && nc[1] >= 3 && nc[2] >= 3) {
+        for (int k = 0; k < 3; ++k) nc[k] = (int)std::floor(s.box[k] / (s.ds_cutoff / reach));
+        const int least = 2 * reach + 1;
+        if (nc[0] >= least && nc[1] >= least && nc[2] >= least) {
             D->g.use_cells = 1;
+            D->g.reach = reach;
             D->g.nc = make_int3(nc[0], nc[1], nc[2]);
         }
     }
@@ -119,15 +122,15 @@ void disp_destroy(mbpol_context* ctx) {
     ctx->disp = nullptr;
 }
 
-void launch_energy_finish(hipStream_t s, int nblocks, const double* eblk, u64* energy);
-
 int disp_evaluate(mbpol_context* ctx, hipStream_t st, u64* energy) {
     Disp* D = ctx->disp;
     const double* pos = ctx->pos.as<double>();
     if (D->g.na == 0) return MBPOL_OK;
     if (D->g.use_cells) {
-        launch_fill_zero(st, D->cell_count.p, sizeof(int) * (D->ncell + 1));
-        launch_fill_zero(st, D->cell_fill.p, sizeof(int) * (D->ncell + 1));
+        FillList L(st);
+        L.add(D->cell_count.p, sizeof(int) * (D->ncell + 1));
+        L.add(D->cell_fill.p, sizeof(int) * (D->ncell + 1));
+        L.launch();
         launch_disp_cells(st, D->g.na, D->act.as<int>(), pos, D->g.L, D->g.nc, D->cell_of.as<int>(), D->cell_count.as<int>());
         if (int e = scan_i32(ctx, D->cell_count.as<int>(), D->cell_start.as<int>(), D->ncell + 1, st)) return e;
         launch_disp_cell_fill(st, D->g.na, D->cell_of.as<int>(), D->cell_start.as<int>(), D->cell_fill.as<int>(),
@@ -142,8 +145,8 @@ int disp_evaluate(mbpol_context* ctx, hipStream_t st, u64* energy) {
                 D->mol.as<int>(), D->c6.as<double>(), D->d6.as<double>(), D->cell_of.as<int>(), D->cell_start.as<int>(),
                 D->members.as<int>(), D->cpos.as<double4>(), ctx->force_fx.as<u64>(), D->eblk.as<double>(),
                 D->cnt.as<unsigned long long>(), ctx->disp_blocks);
-    launch_count_total(st, D->g.na, D->cnt.as<unsigned long long>(), D->npairs.as<unsigned long long>());
-    launch_energy_finish(st, D->g.na, D->eblk.as<double>(), energy);
+    launch_disp_finish(st, D->g.na, D->eblk.as<double>(), D->cnt.as<unsigned long long>(), energy,
+                       D->npairs.as<unsigned long long>());
     return MBPOL_OK;
 }
 

@@ -12,6 +12,7 @@ struct DispGeom {
     double cutoff;  // nm
     d3 L;
     int use_cells;
+    int reach;      // cells searched each way
     int3 nc;
     // independent groups (non-periodic): candidates of active atom a are [gs[a], ge[a]); null = all
     const int *gs, *ge;
@@ -27,7 +28,8 @@ void launch_disp(hipStream_t s, int precision_double, DispGeom g, const int* act
                  const int* mol, const double* c6, const double* d6, const int* cell_of, const int* cell_start,
                  const int* members, const double4* cpos, u64* force, double* eblk, unsigned long long* cnt,
                  int max_blocks = 0);  // max_blocks > 0: capped grid, each wave strides over the atoms
-// cnt: per active atom; launch_count_total sums it into *out
-void launch_count_total(hipStream_t s, int na, const unsigned long long* cnt, unsigned long long* out);
+// the sum of eblk into energy (fixed point) and of the per-atom pair counts into *pairs
+void launch_disp_finish(hipStream_t s, int na, const double* eblk, const unsigned long long* cnt, u64* energy,
+                        unsigned long long* pairs);
 
 }  // namespace mbpol
