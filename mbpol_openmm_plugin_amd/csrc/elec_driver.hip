@@ -62,6 +62,8 @@ static int scratch_address(int device, double** out) {
     return MBPOL_OK;
 }
 
+constexpr size_t kRowBytes = sizeof(int) * kRowSlots * kRowSlotInts;  // device row totals
+
 struct Elec {
     ElecParams P{};
     int n = 0, nw = 0, npol = 0;
@@ -115,7 +117,7 @@ struct Elec {
     bool fuse_spread = true;  // the dipole spreading fused with the z pass (single-axis passes only)
     hipfftHandle plan_f = 0, plan_b = 0;
     bool plans = false;
-    double* h_eps = nullptr;  // pinned, 128 bytes: [0] epsilon, ints from byte 32, a SolveCtl from byte 64
+    double* h_eps = nullptr;  // pinned: [0] epsilon, ints from byte 32, a SolveCtl from byte 64, the row totals from 128
     DevBuf ctl;               // SolveCtl of the running dipole solve
     int last_iters = 0;       // field evaluations of the previous solve (sizes the first batch of steps)
     // row capacities are checked at the end of the evaluation (rows_pending) once
@@ -432,7 +434,7 @@ int elec_create(mbpol_context* ctx) {
     HIP_TRY(E->phi_ind.ensure(sizeof(double) * 10 * std::max(n, 1)));
     HIP_TRY(E->partial.ensure(sizeof(double) * (iterate_blocks(E->npol) + 1)));
     HIP_TRY(E->eps.ensure(sizeof(double) * 4));
-    HIP_TRY(E->maxcnt.ensure(sizeof(int) * 4));
+    HIP_TRY(E->maxcnt.ensure(kRowBytes));
     HIP_TRY(E->eblk.ensure(sizeof(double) * (std::max(energy_blocks(n), sor_blocks(n)) + 1)));
     HIP_TRY(E->cell_of.ensure(sizeof(int) * std::max(n, 1)));
     HIP_TRY(E->members.ensure(sizeof(int) * std::max(n, 1)));
@@ -443,7 +445,7 @@ int elec_create(mbpol_context* ctx) {
     HIP_TRY(E->cell_count.ensure(sizeof(int) * 2));
     HIP_TRY(E->cell_start.ensure(sizeof(int) * 2));
     HIP_TRY(E->cell_fill.ensure(sizeof(int) * 2));
-    HIP_TRY(hipHostMalloc((void**)&E->h_eps, 128, hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void**)&E->h_eps, 128 + kRowBytes, hipHostMallocDefault));
     HIP_TRY(E->ctl.ensure(sizeof(SolveCtl)));
     if (int e = set_groups(ctx)) return e;
     if (!P.pme) set_direct_caps(E);  // direct sum: rows hold every other site (of the group)
@@ -531,6 +533,20 @@ int elec_tuning(const mbpol_context* ctx, const char* name, int* value) {
     return MBPOL_OK;
 }
 
+// the row totals copied from the device, over their slots: longest P row, longest Q
+// row, directed pairs, (polarisable, polarisable) pairs into the ints from byte 32
+static void fold_row_totals(Elec* E) {
+    int* h = reinterpret_cast<int*>(E->h_eps) + 8;
+    const int* slot = reinterpret_cast<const int*>(reinterpret_cast<const char*>(E->h_eps) + 128);
+    h[0] = h[1] = h[2] = h[3] = 0;
+    for (int k = 0; k < kRowSlots; ++k, slot += kRowSlotInts) {
+        h[0] = std::max(h[0], slot[0]);
+        h[1] = std::max(h[1], slot[1]);
+        h[2] += slot[2];
+        h[3] += slot[3];
+    }
+}
+
 static int build_rows(mbpol_context* ctx) {
     Elec* E = ctx->elec;
     hipStream_t st = ctx->stream;
@@ -555,7 +571,7 @@ static int build_rows(mbpol_context* ctx) {
         launch_site_lists(st, n, pos, E->pol.as<double>(), E->P, E->nc, E->reach, E->use_cells, E->cell_of.as<int>(),
                           E->cell_start.as<int>(), E->cpos.as<double4>(), E->capP, E->capQ, E->nbP.as<int>(),
                           E->cntP.as<int>(), E->nbQ.as<int>(), E->cntQ.as<int>(), E->maxcnt.as<int>());
-        HIP_TRY(hipMemcpyAsync(h, E->maxcnt.p, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipMemcpyAsync(reinterpret_cast<char*>(E->h_eps) + 128, E->maxcnt.p, kRowBytes, hipMemcpyDeviceToHost, st));
         return MBPOL_OK;
     };
     E->rows_pending = false;
@@ -567,9 +583,10 @@ static int build_rows(mbpol_context* ctx) {
         if (int e = build()) return e;
         E->rows_pending = true;
     } else for (int attempt = 0; attempt < 2; ++attempt) {
-        launch_fill_zero(st, E->maxcnt.p, sizeof(int) * 4);
+        launch_fill_zero(st, E->maxcnt.p, kRowBytes);
         if (int e = build()) return e;
         HIP_TRY(hipStreamSynchronize(st));
+        fold_row_totals(E);
         if (h[0] <= E->capP && h[1] <= E->capQ) break;
         if (attempt == 1) return set_error(MBPOL_ERR_HIP, "electrostatics neighbour rows overflowed twice");
         E->capP = std::max(E->capP, (h[0] + h[0] / 4 + 63) / 32 * 32);
@@ -904,6 +921,7 @@ int elec_rows_check(mbpol_context* ctx, bool& redo) {
     if (!E || !E->rows_pending) return MBPOL_OK;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     E->rows_pending = false;
+    fold_row_totals(E);
     const int* h = reinterpret_cast<const int*>(E->h_eps) + 8;
     if (h[0] > E->capP || h[1] > E->capQ) {
         E->capP = std::max(E->capP, (h[0] + h[0] / 4 + 63) / 32 * 32);
@@ -978,7 +996,7 @@ int elec_evaluate(mbpol_context* ctx, u64* energy, const std::function<int()>& a
             L.add(E->cell_count.p, sizeof(int) * (ncell + 1));
             L.add(E->cell_fill.p, sizeof(int) * (ncell + 1));
         }
-        L.add(E->maxcnt.p, sizeof(int) * 4);
+        L.add(E->maxcnt.p, kRowBytes);
         L.add(E->efix.p, sizeof(double) * 3 * n);
         if (P.pme) {
             const size_t rows2 = 2 * (size_t)P.grid.x * P.grid.y;

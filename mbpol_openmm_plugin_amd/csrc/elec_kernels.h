@@ -45,6 +45,10 @@ struct SolveCtl {
     double eps;      // the reference's measure at the last test
 };
 
+// row maxima and totals: kRowSlots sets of 4 ints (longest P row, longest Q row, directed pairs, pol-pol pairs),
+// a cache line apart
+constexpr int kRowSlots = 32, kRowSlotInts = 16;
+
 void launch_site_charges_copy(hipStream_t s, int n, const double* q0, double* q);
 // dst = src (n doubles) when ctl records a converged stop, else nothing
 void launch_copy_if_converged(hipStream_t s, long long n, const SolveCtl* ctl, const double* src, double* dst);

@@ -250,7 +250,10 @@ __device__ __forceinline__ void row_consider(int i, double xi, double yi, double
     cQ += __popcll(bQ);
 }
 
-// row maxima and totals: combined in LDS, one set of global atomics per block
+// row maxima and totals: combined in LDS, one set of global atomics per block, on one
+// of kRowSlots cache lines (on a single line the atomics of 4300 blocks took most of
+// the pass's 205 us for 68,800 sites of 512 clusters; 37 now.  With cells 230 -> 194
+// us for 55,296 sites, 93 -> 67 for 16,384)
 struct RowTotals {
     int v[4];
 };
@@ -262,10 +265,11 @@ __device__ __forceinline__ void row_totals_add(RowTotals& red, int cP, int cQ, b
 }
 __device__ __forceinline__ void row_totals_out(const RowTotals& red, int* __restrict__ maxcnt) {
     if (threadIdx.x == 0) {
-        atomicMax(&maxcnt[0], red.v[0]);
-        atomicMax(&maxcnt[1], red.v[1]);
-        atomicAdd(&maxcnt[2], red.v[2]);
-        atomicAdd(&maxcnt[3], red.v[3]);
+        int* slot = maxcnt + kRowSlotInts * (blockIdx.x % kRowSlots);
+        atomicMax(&slot[0], red.v[0]);
+        atomicMax(&slot[1], red.v[1]);
+        atomicAdd(&slot[2], red.v[2]);
+        atomicAdd(&slot[3], red.v[3]);
     }
 }
 
@@ -320,7 +324,7 @@ __global__ void k_site_pack(int n, const int* __restrict__ members, const double
 // loaded ahead.
 // What bounds it: the traffic of the candidates (1500 entries of 32 bytes a site)
 // with one site a wave -- 220 us for 16,384 sites, 127 us for 8788; with 16 or 32
-// lanes a site walking range after range, latency, 127 us for both; now 93 and 74 us, bound
+// lanes a site walking range after range, latency, 127 us for both; now 67 and 70 us, bound
 // by the instructions of the tests (about 45 for 64 candidates and a site).
 constexpr int kRowSites = 4;
 __global__ void __launch_bounds__(256) k_site_lists_cells(int n, ElecParams P, int3 nc, int reach,
