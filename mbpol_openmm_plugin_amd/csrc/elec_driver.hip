@@ -101,7 +101,7 @@ struct Elec {
     // independent groups: site ranges, per-group preconditioner blocks and site counts, per-block
     // |alpha r|^2, per-site energies
     int ngroups = 0, cap_grp_pol = 0, cap_grp_other = 0;
-    DevBuf g_site_s, g_site_e, g_blk_start, g_nsites, g_blk_ee, g_esite;
+    DevBuf g_site_s, g_site_e, g_blk_start, g_nsites, g_blk_ee, g_eps, g_esite;
     double* mu_cur = nullptr;  // dipoles of the last evaluate
     DevBuf phi_fix, phi_ind, fsite, V, eblk;
     // PME
@@ -374,6 +374,7 @@ static int set_groups(mbpol_context* ctx) {
     if (int e = up(ctx->stream, E->g_blk_start, bs)) return e;
     if (int e = up(ctx->stream, E->g_nsites, ns)) return e;
     HIP_TRY(E->g_blk_ee.ensure(sizeof(double) * std::max(E->nblk, 1)));
+    HIP_TRY(E->g_eps.ensure(sizeof(double) * G));
     HIP_TRY(E->g_esite.ensure(sizeof(double) * std::max(E->n, 1)));
     E->P.gs = E->g_site_s.as<int>();
     E->P.ge = E->g_site_e.as<int>();
@@ -784,7 +785,8 @@ static int solve_pcg(mbpol_context* ctx, double* x, double self_term, SolveCtl& 
     const PrecondBlocks B{E->nblk, E->blk_start.as<int>(), E->blk_site.as<int>()};
     double* minv = E->minv.as<double>();
     // independent groups: convergence of the worst group
-    const GroupConv gc{E->ngroups, E->g_blk_start.as<int>(), E->g_nsites.as<int>(), E->g_blk_ee.as<double>()};
+    const GroupConv gc{E->ngroups, E->g_blk_start.as<int>(), E->g_nsites.as<int>(), E->g_blk_ee.as<double>(),
+                       E->g_eps.as<double>()};
     double* blk_ee = E->ngroups ? E->g_blk_ee.as<double>() : nullptr;
     auto field = [&](const double* v, int mode, double* out) -> int {
         if (P.pme)

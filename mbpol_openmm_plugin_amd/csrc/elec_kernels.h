@@ -91,6 +91,7 @@ struct GroupConv {
     const int* blk_start;
     const int* nsites;  // sites of each group (all of them, as the reference's measure counts)
     const double* blk_ee;
+    double* eps;  // scratch: the measure of every group
 };
 
 // preconditioned conjugate gradients on A mu = E_fix, A = diag(1/alpha) - T (see kernels_elec.hip)
