@@ -42,16 +42,9 @@ FLOPS_PER_DIMER = 31.0e3
 # HBM bytes per launch from rocprofv3 FETCH_SIZE + WRITE_SIZE counters on this
 # workload, calibrated against the runtime's plain copy kernel in the same runs
 # (FETCH_SIZE x 1.885, WRITE_SIZE x 1.000; the runs are summarised under
-# profiles/); kernels not listed report null
+# profiles/); kernels not listed (not counted since they were last changed) report null
 MEASURED_TRAFFIC = {
     'elec_iterate': 85816165,
-    'spread_fft_z': 84248140,
-    'fft_z_r2c': 28177550,
-    'fft_y': 25651329,
-    'fft_x_conv': 38354591,
-    'fft_z_c2r': 25337943,
-    'threebody': 114310400,
-    'twobody': 58527178,
 }
 
 
@@ -82,6 +75,7 @@ def kernel_models(stats, grid, nsites, npol):
     (kind, amount, bound, peak, unit)."""
     K0, K1, K2 = grid
     ngrid, nhalf = K0 * K1 * K2, K0 * K1 * (K2 // 2 + 1)
+    spread = (K0 * K1 + 1) * 4 + nsites * (25 * 32 + 80) + npol * 24
     return {
         'threebody': ('flops', FLOPS_PER_TRIMER * stats['num_trimers'], 'valu', PEAK_FP64_TFLOPS, 'TFLOP/s'),
         'twobody': ('flops', FLOPS_PER_DIMER * stats['num_dimers'], 'valu', PEAK_FP64_TFLOPS, 'TFLOP/s'),
@@ -91,12 +85,12 @@ def kernel_models(stats, grid, nsites, npol):
         # site once, the site's own vector / polarisability / row length and its result
         'elec_iterate': ('bytes', stats['num_pol_pairs'] * 20 + ngrid * 8 + nsites * 48 + npol * (24 + 24 + 8 + 4 + 4),
                          'hbm', PEAK_HBM_GBS, 'GB/s'),
-        # row starts, entries (site + 3 FP64 coefficients), dipoles, grid write
-        'pme_spread': ('bytes', (ngrid + 1) * 4 + npol * 125 * 28 + npol * 24 + ngrid * 8, 'hbm', PEAK_HBM_GBS, 'GB/s'),
+        # line starts, 25 entries per site (site, first z, 3 FP64 weights), its z spline values and
+        # derivatives, dipoles, grid write
+        'pme_spread': ('bytes', spread + ngrid * 8, 'hbm', PEAK_HBM_GBS, 'GB/s'),
         'fft_z_r2c': ('bytes', ngrid * 8 + nhalf * 16, 'hbm', PEAK_HBM_GBS, 'GB/s'),
-        # the dipole spreading fused with the z pass: row starts, entries, dipoles, half spectrum write
-        'spread_fft_z': ('bytes', (ngrid + 1) * 4 + npol * 125 * 28 + npol * 24 + nhalf * 16, 'hbm', PEAK_HBM_GBS,
-                         'GB/s'),
+        # the spreading fused with the z pass: the same reads, half spectrum write
+        'spread_fft_z': ('bytes', spread + nhalf * 16, 'hbm', PEAK_HBM_GBS, 'GB/s'),
         'fft_y': ('bytes', nhalf * 32, 'hbm', PEAK_HBM_GBS, 'GB/s'),
         'fft_x_conv': ('bytes', nhalf * 40, 'hbm', PEAK_HBM_GBS, 'GB/s'),
         'fft_z_c2r': ('bytes', nhalf * 16 + ngrid * 8, 'hbm', PEAK_HBM_GBS, 'GB/s'),

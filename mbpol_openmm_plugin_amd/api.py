@@ -550,7 +550,7 @@ class Context:
         _check(library().mbpol_context_set_solver(self._h, SOLVERS[solver]))
 
     def getTuning(self, name):
-        """Launch shape picked by the context's autotuning ('site_lanes'), a grid cap
+        """Lanes that build the electrostatics rows ('site_lanes': 64 with cells, 16 without), a grid cap
         ('pip_blocks', 'pip3_blocks', 'disp_blocks'), the 2- and 3-body kernels ('pip2_kernel', 'pip3_kernel':
         0 the loop over the relabelling group, 1 term by term),
         a capacity ('row_capacity_pol', 'row_capacity_other', 'dimer_capacity',
