@@ -330,10 +330,11 @@ class ThreeParticleAverageSite:
 
 
 class System:
+    _vsite_arrays = None  # the virtual sites as arrays, with what they were made from (computeVirtualSites)
+
     def __init__(self):
         self._masses = []
         self._vsites = {}
-        self._vsite_arrays = None  # the virtual sites as arrays, with what they were made from (computeVirtualSites)
         self._forces = []
         self._box = None
         self._groups = None
@@ -406,20 +407,36 @@ class System:
         have to be placed one by one."""
         sites = self._vsites.values()
         made_from = (list(self._vsites), [v.particles for v in sites], [v.weights for v in sites])
-        if self._vsite_arrays is None or self._vsite_arrays[0] != made_from:
+        kept = self._vsite_arrays
+        try:
+            same = kept is not None and kept[0] == made_from
+        except ValueError:  # a site holds an array, which does not compare to one truth value
+            same = False
+        if not same:
             index, parents, weights = made_from
-            table = None
-            if all(len(p) == 3 and len(w) == 3 for p, w in zip(parents, weights)):
-                ip = np.array(parents, dtype=np.int64).reshape(-1, 3)
-                n = self.getNumParticles()
-                at = np.array(index, dtype=np.int64)
-                # negative indices count from the end, as in the loop
-                if not np.isin(np.where(ip < 0, ip + n, ip), np.where(at < 0, at + n, at)).any():
-                    table = (at, ip, np.array(weights, dtype=np.float64).reshape(-1, 3))
             # kept as tuples: a list changed in place does not compare equal
             made_from = (index, [tuple(p) for p in parents], [tuple(w) for w in weights])
-            self._vsite_arrays = (made_from, table)
-        return self._vsite_arrays[1]
+            kept = self._vsite_arrays = (made_from, self._plain_table(*made_from))
+        return kept[1]
+
+    @staticmethod
+    def _plain_table(index, parents, weights):
+        """The arrays of sites that all have three parents and weights, plain numbers, none counted from the
+        end and none a virtual site itself; None otherwise: the loop takes other forms (weights per
+        coordinate, wider floats, negative indices) or refuses them, as an array conversion would not."""
+        if any(len(t) != 3 for t in parents) or any(len(t) != 3 for t in weights):
+            return None
+        parent, weight = [v for t in parents for v in t], [v for t in weights for v in t]
+        if not set(map(type, index + parent)) <= {int} or not all(t is int or issubclass(t, float)
+                                                                  for t in set(map(type, weight))):
+            return None
+        if index and (min(index + parent) < 0 or max(index + parent) >= 2 ** 63 or
+                      any(type(w) is int and abs(w) > 2 ** 53 for w in weight)):
+            return None
+        if not set(index).isdisjoint(parent):
+            return None
+        return (np.array(index, dtype=np.int64), np.array(parents, dtype=np.int64).reshape(-1, 3),
+                np.array(weights, dtype=np.float64).reshape(-1, 3))
 
 
 class State:
