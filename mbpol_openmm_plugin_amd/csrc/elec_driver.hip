@@ -114,6 +114,7 @@ struct Elec {
     DevBuf tw[3];
     bool lds_fft = false;
     bool plane_fft = false;  // z and y passes fused per x plane
+    int nseg = 1;             // segments of a line in the spreading table (1 where the z pass takes whole lines)
     bool fuse_spread = true;  // the dipole spreading fused with the z pass (single-axis passes only)
     hipfftHandle plan_f = 0, plan_b = 0;
     bool plans = false;
@@ -381,6 +382,11 @@ static int set_groups(mbpol_context* ctx) {
     return MBPOL_OK;
 }
 
+// whether the spreading and a dense z pass of the single-axis passes run in one kernel
+static bool spread_fused(const Elec* E) {
+    return E->lds_fft && !E->plane_fft && E->fuse_spread && E->fft.ax[2].dense;
+}
+
 int elec_create(mbpol_context* ctx) {
     const mbpol_system& s = ctx->sys;
     Elec* E = new Elec();
@@ -480,8 +486,11 @@ int elec_create(mbpol_context* ctx) {
         if (int e = up(ctx->stream, E->bz, bspline_moduli(grid[2]))) return e;
         HIP_TRY(E->g0tab.ensure(sizeof(int) * 3 * std::max(n, 1)));
         HIP_TRY(E->sptab.ensure(sizeof(double) * 30 * std::max(n, 1)));
-        for (DevBuf* b : {&E->rowcount, &E->rowstart, &E->rowfill})
-            HIP_TRY(b->ensure(sizeof(int) * (2 * (size_t)grid[0] * grid[1] + 1)));
+        E->nseg = spread_fused(E) ? 1 : spread_segments(grid[2]);
+        const size_t rows2 = 2 * (size_t)grid[0] * grid[1] * E->nseg;
+        if (rows2 >= (1u << 31))
+            return set_error(MBPOL_ERR_INVALID_ARGUMENT, "PME grid %d x %d x %d is too large", grid[0], grid[1], grid[2]);
+        for (DevBuf* b : {&E->rowcount, &E->rowstart, &E->rowfill}) HIP_TRY(b->ensure(sizeof(int) * (rows2 + 1)));
         if (lds) {
             for (int d = 0; d < 3; ++d) {
                 const int m = grid[d];
@@ -606,14 +615,14 @@ static int build_rows(mbpol_context* ctx) {
     if (E->P.pme) {
         launch_site_spline_table(st, n, pos, E->P, E->g0tab.as<int>(), E->sptab.as<double>());
         // spreading table
-        const int rows2 = 2 * E->P.grid.x * E->P.grid.y;
+        const int rows2 = 2 * E->P.grid.x * E->P.grid.y * E->nseg;
         const size_t nent = (size_t)n * 25;
         HIP_TRY(E->ecode.ensure(sizeof(int) * std::max<size_t>(nent, 1)));
         HIP_TRY(E->esz.ensure(sizeof(int2) * std::max<size_t>(nent, 1)));
         HIP_TRY(E->ecoef.ensure(sizeof(double) * 3 * std::max<size_t>(nent, 1)));
         auto table = [&](int stage) {
             launch_line_table(st, stage, n, E->g0tab.as<int>(), E->sptab.as<double>(), E->pol.as<double>(),
-                              E->q.as<double>(), E->P, E->rowcount.as<int>(), E->rowstart.as<int>(),
+                              E->q.as<double>(), E->P, E->nseg, E->rowcount.as<int>(), E->rowstart.as<int>(),
                               E->rowfill.as<int>(), E->ecode.as<int>(), E->esz.as<int2>(), E->ecoef.as<double>());
         };
         table(0);
@@ -629,10 +638,9 @@ static int pme_grid(mbpol_context* ctx, int mode, const double* mu, const int* s
     hipStream_t st = ctx->stream;
     const ElecParams& P = E->P;
     const size_t nhalf = (size_t)P.grid.x * P.grid.y * (P.grid.z / 2 + 1);
-    const LineTable T{P.grid.x * P.grid.y, P.grid.z, E->rowstart.as<int>(), E->esz.as<int2>(), E->ecoef.as<double>(),
+    const LineTable T{P.grid.x * P.grid.y, P.grid.z, E->nseg, E->rowstart.as<int>(), E->esz.as<int2>(), E->ecoef.as<double>(),
                       E->sptab.as<double>(), P.grid.z * P.inv_box.z};
-    // the spreading and a dense z pass of the single-axis passes in one kernel
-    const bool fused = E->lds_fft && !E->plane_fft && E->fuse_spread && E->fft.ax[2].dense;
+    const bool fused = spread_fused(E);
     if (fused) {
         const int cat = mode == 0 ? T_FFT_Z_R2C : T_SPREAD_FFT_Z;
         const KEvents ev = timer_kernel(ctx, cat);
@@ -1001,7 +1009,7 @@ int elec_evaluate(mbpol_context* ctx, u64* energy, const std::function<int()>& a
         L.add(E->maxcnt.p, kRowBytes);
         L.add(E->efix.p, sizeof(double) * 3 * n);
         if (P.pme) {
-            const size_t rows2 = 2 * (size_t)P.grid.x * P.grid.y;
+            const size_t rows2 = 2 * (size_t)P.grid.x * P.grid.y * E->nseg;
             L.add(E->rowcount.p, sizeof(int) * (rows2 + 1));
             L.add(E->rowfill.p, sizeof(int) * (rows2 + 1));
         }

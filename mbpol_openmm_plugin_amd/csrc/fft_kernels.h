@@ -34,16 +34,27 @@ constexpr int kFftMaxLength = 1024;
 // stop: when non-null and *stop != 0 at launch, the pass does nothing (a dipole solve that has converged)
 void launch_fft_z_r2c(hipStream_t s, const PmeFft& F, const double* real, double2* H, const KEvents& ev,
                       const int* stop = nullptr);
-// The spreading table by grid line (kernels_elec.hip): rows 0 .. nlines - 1 the polarisable sites of a line,
-// rows nlines .. 2 nlines - 1 its other charged sites
+// The spreading table by grid line (kernels_elec.hip): rows 0 .. nseg nlines - 1 the polarisable sites of the
+// lines' segments, line by line, rows nseg nlines .. 2 nseg nlines - 1 the other charged sites
 struct LineTable {
     int nlines, nz;  // lines (x, y), points of a line
+    int nseg;        // segments a line's points are cut into
     const int* start;
     const int2* sz;      // site, first z
     const double* coef;  // 3 per entry
     const double* sptab; // z splines: sptab[30 site + 20 ..]
     double scale_z;      // K_z / L_z
 };
+// first point of segment s of nz points in nseg segments whose lengths differ by at most one
+__host__ __device__ inline int segment_start(int s, int nz, int nseg) { return (int)((long long)s * nz / nseg); }
+// the segment that point z lies in: the last one that starts at or before it
+__host__ __device__ inline int segment_of(int z, int nz, int nseg) {
+    return (int)(((long long)(z + 1) * nseg - 1) / nz);
+}
+// Segments of a line of nz points: none shorter than 64 points (a site's 5 then
+// reach into the next one at most), none longer than 127 (17 KB of LDS).
+constexpr int kSegmentPoints = 64;
+inline int spread_segments(int nz) { return nz < 2 * kSegmentPoints ? 1 : nz / kSegmentPoints; }
 // spreads charges (w = q) or dipoles (w = mu) onto the real grid, or straight into the forward z pass (dense z only)
 void launch_spread_lines(hipStream_t s, const LineTable& T, bool charges, const double* w, double* real,
                          const KEvents& ev, const int* stop = nullptr);

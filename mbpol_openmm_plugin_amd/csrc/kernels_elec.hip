@@ -17,6 +17,7 @@
 
 #include "device_common.h"
 #include "elec_kernels.h"
+#include "fft_kernels.h"
 
 namespace mbpol {
 using namespace mbpol_params;
@@ -660,51 +661,52 @@ __global__ void k_site_spline_table(int n, const double* __restrict__ pos, ElecP
 // the grids of the charges and of every iteration's dipoles are linear in them:
 // site i adds (mu_x c0 + mu_y c1) v0[z] + mu_z K_z/L_z c2 v1[z], or q c2 v0[z], to 5
 // points of each of 25 (x, y) lines, with c = (K_x/L_x t1 u0, K_y/L_y t0 u1, t0 u0)
-// and the z splines v0, v1 of the site.  The table lists, line by line, the sites
-// (in index order: every sum has a fixed order) with their first z and c: rows
-// 0 .. nlines-1 the polarisable sites, rows nlines .. 2 nlines-1 the other charged
-// ones.  A seventh of the memory of a table by grid point (32 bytes for 5 points
+// and the z splines v0, v1 of the site.  The table lists, line by line and in a line
+// segment by segment of its points (nseg, by the first z), the sites (in index order:
+// every sum has a fixed order) with their first z and c: the lines' rows first for the
+// polarisable sites, then for the other charged ones.  A seventh of the memory of a table by grid point (32 bytes for 5 points
 // against 28 for each), and of the work to build it.
 // ---------------------------------------------------------------------------
 // row of entry c (0..24) of site i; -1 when the site adds nothing
 __device__ __forceinline__ int line_row(int i, int c, const int* __restrict__ g0tab, const double* __restrict__ pol,
-                                        const double* __restrict__ q, const ElecParams& P) {
+                                        const double* __restrict__ q, const ElecParams& P, int nseg) {
     const bool polarisable = pol[i] != 0.0;
     if (!polarisable && q[i] == 0.0) return -1;
     const int gx = wrapg(g0tab[3 * i] + c / 5, P.grid.x), gy = wrapg(g0tab[3 * i + 1] + c % 5, P.grid.y);
-    return (polarisable ? 0 : P.grid.x * P.grid.y) + gx * P.grid.y + gy;
+    const int line = (polarisable ? 0 : P.grid.x * P.grid.y) + gx * P.grid.y + gy;
+    return nseg == 1 ? line : line * nseg + segment_of(g0tab[3 * i + 2], P.grid.z, nseg);
 }
 
 __global__ void k_line_count(int n, const int* __restrict__ g0tab, const double* __restrict__ pol,
-                             const double* __restrict__ q, ElecParams P, int* __restrict__ rowcount) {
+                             const double* __restrict__ q, ElecParams P, int nseg, int* __restrict__ rowcount) {
     critical_path_wave();
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= 25 * n) return;
-    const int r = line_row(t / 25, t % 25, g0tab, pol, q, P);
+    const int r = line_row(t / 25, t % 25, g0tab, pol, q, P, nseg);
     if (r >= 0) atomicAdd(&rowcount[r], 1);
 }
 
 // entry codes 25 i + c into their rows, in arbitrary order within a row
 __global__ void k_line_fill(int n, const int* __restrict__ g0tab, const double* __restrict__ pol,
-                            const double* __restrict__ q, ElecParams P, const int* __restrict__ rowstart,
+                            const double* __restrict__ q, ElecParams P, int nseg, const int* __restrict__ rowstart,
                             int* __restrict__ fill, int* __restrict__ code) {
     critical_path_wave();
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= 25 * n) return;
-    const int r = line_row(t / 25, t % 25, g0tab, pol, q, P);
+    const int r = line_row(t / 25, t % 25, g0tab, pol, q, P, nseg);
     if (r >= 0) code[rowstart[r] + atomicAdd(&fill[r], 1)] = t;
 }
 
 // the entries in site order: an entry's place is the number of smaller codes in its row
 __global__ void k_line_sort(int n, const int* __restrict__ g0tab, const double* __restrict__ sptab,
-                            const double* __restrict__ pol, const double* __restrict__ q, ElecParams P,
+                            const double* __restrict__ pol, const double* __restrict__ q, ElecParams P, int nseg,
                             const int* __restrict__ rowstart, const int* __restrict__ code, int2* __restrict__ sz,
                             double* __restrict__ coef) {
     critical_path_wave();
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= rowstart[2 * P.grid.x * P.grid.y]) return;
+    if (s >= rowstart[2 * P.grid.x * P.grid.y * nseg]) return;
     const int t = code[s], i = t / 25, c = t % 25;
-    const int r = line_row(i, c, g0tab, pol, q, P);
+    const int r = line_row(i, c, g0tab, pol, q, P, nseg);
     const int b = rowstart[r], e = rowstart[r + 1];
     int at = b;
     for (int k = b; k < e; ++k) at += code[k] < t ? 1 : 0;
@@ -1615,16 +1617,16 @@ void launch_site_spline_table(hipStream_t s, int n, const double* pos, ElecParam
     hipLaunchKernelGGL(k_site_spline_table, nblk(n, 128), 128, 0, s, n, pos, P, g0tab, sptab);
 }
 void launch_line_table(hipStream_t s, int stage, int n, const int* g0tab, const double* sptab, const double* pol,
-                       const double* q, ElecParams P, int* rowcount, const int* rowstart, int* rowfill, int* code,
+                       const double* q, ElecParams P, int nseg, int* rowcount, const int* rowstart, int* rowfill, int* code,
                        int2* sz, double* coef) {
     if (n <= 0) return;
     const int blocks = nblk(25LL * n, 256);
     if (stage == 0) {
-        hipLaunchKernelGGL(k_line_count, blocks, 256, 0, s, n, g0tab, pol, q, P, rowcount);
+        hipLaunchKernelGGL(k_line_count, blocks, 256, 0, s, n, g0tab, pol, q, P, nseg, rowcount);
         return;
     }
-    hipLaunchKernelGGL(k_line_fill, blocks, 256, 0, s, n, g0tab, pol, q, P, rowstart, rowfill, code);
-    hipLaunchKernelGGL(k_line_sort, blocks, 256, 0, s, n, g0tab, sptab, pol, q, P, rowstart, code, sz, coef);
+    hipLaunchKernelGGL(k_line_fill, blocks, 256, 0, s, n, g0tab, pol, q, P, nseg, rowstart, rowfill, code);
+    hipLaunchKernelGGL(k_line_sort, blocks, 256, 0, s, n, g0tab, sptab, pol, q, P, nseg, rowstart, code, sz, coef);
 }
 void launch_convolve(hipStream_t s, size_t nhalf, const double* influence, double2* spec) {
     hipLaunchKernelGGL(k_convolve, nblk(nhalf, 256), 256, 0, s, nhalf, influence, spec);
