@@ -41,9 +41,10 @@ using namespace mbpol_params;
 typedef PIP_REAL real;
 typedef v3<real> vr;
 
-// image_to by products with 1/L: the image index differs from the one the quotient
-// gives only where a separation is within rounding of half the box, at or beyond
-// every cutoff, where the switches are zero
+// image_to by products with 1/L, for a hydrogen about its own oxygen: the image index differs from the one
+// the quotient gives only where a separation is within rounding of half the box, which no O-H distance is.
+// Oxygens take image_to: a third molecule half a box from the first has a switch of zero with it, but which
+// of its images is taken decides its distance from the second.
 __device__ __forceinline__ d3 image_near(const d3& ref, const d3& p, const d3& L, const d3& iL) {
     return d3{p.x + L.x * floor((ref.x - p.x) * iL.x + 0.5), p.y + L.y * floor((ref.y - p.y) * iL.y + 0.5),
               p.z + L.z * floor((ref.z - p.z) * iL.z + 0.5)};
@@ -163,7 +164,7 @@ __device__ __forceinline__ bool dimer_geometry(long long t, const int2* __restri
         const d3 iL{1.0 / boxA.x, 1.0 / boxA.y, 1.0 / boxA.z};
         P[1] = image_near(P[0], P[1], boxA, iL);
         P[2] = image_near(P[0], P[2], boxA, iL);
-        P[3] = image_near(P[0], P[3], boxA, iL);
+        P[3] = image_to(P[0], P[3], boxA);
         P[4] = image_near(P[3], P[4], boxA, iL);
         P[5] = image_near(P[3], P[5], boxA, iL);
     }
@@ -207,7 +208,7 @@ __device__ __forceinline__ bool unit_geometry(long long t, const int2* __restric
         const d3 L{box.x * 10., box.y * 10., box.z * 10.}, iL{1.0 / L.x, 1.0 / L.y, 1.0 / L.z};
         P[1] = image_near(P[0], P[1], L, iL);
         P[2] = image_near(P[0], P[2], L, iL);
-        P[3] = image_near(P[0], P[3], L, iL);
+        P[3] = image_to(P[0], P[3], L);
         P[4] = image_near(P[3], P[4], L, iL);
         P[5] = image_near(P[3], P[5], L, iL);
     }
@@ -461,10 +462,10 @@ __device__ __forceinline__ bool trimer_geometry(long long t, const int* __restri
         const d3 iL{1.0 / box.x, 1.0 / box.y, 1.0 / box.z};
         P[1] = image_near(P[0], P[1], box, iL);
         P[2] = image_near(P[0], P[2], box, iL);
-        P[3] = image_near(P[0], P[3], box, iL);
+        P[3] = image_to(P[0], P[3], box);
         P[4] = image_near(P[3], P[4], box, iL);
         P[5] = image_near(P[3], P[5], box, iL);
-        P[6] = image_near(P[0], P[6], box, iL);
+        P[6] = image_to(P[0], P[6], box);
         P[7] = image_near(P[6], P[7], box, iL);
         P[8] = image_near(P[6], P[8], box, iL);
     }
@@ -495,10 +496,10 @@ __device__ __forceinline__ bool unit_geometry(long long t, const int* __restrict
         const d3 iL{1.0 / box.x, 1.0 / box.y, 1.0 / box.z};
         P[1] = image_near(P[0], P[1], box, iL);
         P[2] = image_near(P[0], P[2], box, iL);
-        P[3] = image_near(P[0], P[3], box, iL);
+        P[3] = image_to(P[0], P[3], box);
         P[4] = image_near(P[3], P[4], box, iL);
         P[5] = image_near(P[3], P[5], box, iL);
-        P[6] = image_near(P[0], P[6], box, iL);
+        P[6] = image_to(P[0], P[6], box);
         P[7] = image_near(P[6], P[7], box, iL);
         P[8] = image_near(P[6], P[8], box, iL);
     }
