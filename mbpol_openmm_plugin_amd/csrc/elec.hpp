@@ -9,6 +9,9 @@ namespace mbpol {
 constexpr double kFixInvHost = 1.0 / 4294967296.0;
 
 int set_error(int code, const char* fmt, ...);
+// MBPOL_OK, or the error of a kernel that this thread could not launch since the last call (a launch returns
+// nothing itself, and waiting for the stream does not report it)
+int launch_status();
 // exclusive scans on stream s (nullptr: the context's main stream)
 int scan_i32(mbpol_context* ctx, const int* in, int* out, int n, hipStream_t s = nullptr);
 int scan_i64(mbpol_context* ctx, const long long* in, long long* out, int n, hipStream_t s = nullptr);

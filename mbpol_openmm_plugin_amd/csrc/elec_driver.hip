@@ -1252,8 +1252,10 @@ int mbpol_context_get_electrostatic_potential(mbpol_context* ctx, int32_t npoint
     HIP_TRY(out.ensure(sizeof(double) * npoints));
     HIP_TRY(copy_on(ctx->stream, pts.p, points, sizeof(double) * 3 * npoints));
     Elec* E = ctx->elec;
+    (void)hipGetLastError();
     launch_potential_at_points(ctx->stream, npoints, pts.as<double>(), E->n, ctx->pos.as<double>(), E->q.as<double>(),
                                E->mu_cur, E->P, out.as<double>());
+    if (int e = launch_status()) return e;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(copy_on(ctx->stream, potential, out.p, sizeof(double) * npoints));
     return MBPOL_OK;
@@ -1279,8 +1281,10 @@ int mbpol_context_get_electrostatic_potential_noalloc(mbpol_context* ctx, int32_
     double* out = sc + 3 * (size_t)kScratchPoints;
     Elec* E = ctx->elec;
     HIP_TRY(hipMemcpyAsync(pts, points, sizeof(double) * 3 * npoints, hipMemcpyHostToDevice, ctx->stream));
+    (void)hipGetLastError();
     launch_potential_at_points(ctx->stream, npoints, pts, E->n, ctx->pos.as<double>(), E->q.as<double>(), E->mu_cur,
                                E->P, out);
+    if (int e = launch_status()) return e;
     HIP_TRY(hipMemcpyAsync(potential, out, sizeof(double) * npoints, hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     return MBPOL_OK;
@@ -1296,8 +1300,10 @@ int mbpol_context_get_system_electrostatics_moments(mbpol_context* ctx, const do
     HIP_TRY(m.ensure(sizeof(double) * E->n));
     HIP_TRY(out.ensure(sizeof(double) * 13));
     HIP_TRY(copy_on(ctx->stream, m.p, masses, sizeof(double) * E->n));
+    (void)hipGetLastError();
     launch_system_moments(ctx->stream, E->n, ctx->pos.as<double>(), E->q.as<double>(), E->mu_cur, m.as<double>(),
                           out.as<double>());
+    if (int e = launch_status()) return e;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     HIP_TRY(copy_on(ctx->stream, moments, out.p, sizeof(double) * 13));
     return MBPOL_OK;

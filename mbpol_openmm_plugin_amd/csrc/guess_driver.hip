@@ -542,11 +542,13 @@ int mbpol_md_step(mbpol_md* md, int32_t nsteps, double* energies_out, double* ki
     const double* im = md->inv_mass.as<double>();
     double* v = md->vel.as<double>();
     const double h = 0.5 * md->dt, a = std::exp(-md->gamma * md->dt), kT = kBoltzmann * md->T;
+    (void)hipGetLastError();
     for (int s = 0; s < nsteps; ++s) {
         launch_md_kick(st, n, f, im, h, v);
         launch_md_drift(st, n, v, im, h, x);
         launch_md_thermostat(st, n, im, a, kT, md->seed, md->step++, v);
         launch_md_drift(st, n, v, im, h, x);
+        if (int e = launch_status()) return e;
         if (int e = mbpol_context_evaluate_resident(ctx, md->last_e, md->components)) return e;
         launch_md_kick(st, n, f, im, h, v);
     }
@@ -558,7 +560,7 @@ int mbpol_md_step(mbpol_md* md, int32_t nsteps, double* energies_out, double* ki
     } else {
         HIP_TRY(hipStreamSynchronize(st));
     }
-    return MBPOL_OK;
+    return launch_status();
 }
 
 int mbpol_md_get_positions(const mbpol_md* md, double* positions) {

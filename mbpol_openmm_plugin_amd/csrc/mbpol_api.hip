@@ -51,6 +51,11 @@ int mbpol::set_error(int code, const char* fmt, ...) {
         if (_e != hipSuccess) return set_error(MBPOL_ERR_HIP, "%s: %s", #expr, hipGetErrorString(_e)); \
     } while (0)
 
+int mbpol::launch_status() {
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? MBPOL_OK : set_error(MBPOL_ERR_HIP, "a kernel could not be launched: %s", hipGetErrorString(e));
+}
+
 DevBuf::~DevBuf() {
     if (p) (void)hipFree(p);
 }
@@ -964,6 +969,7 @@ static int enqueue_evaluation(mbpol_context* ctx, double* forces_dev_out, uint32
     u64* F = ctx->force_fx.as<u64>();
     u64* E = ctx->energy_fx.as<u64>();
     double* pos = ctx->pos.as<double>();
+    (void)hipGetLastError();  // an earlier error of the caller's is not this evaluation's
     {
         FillList L(st);
         L.add(F, sizeof(u64) * 3 * s.n);
@@ -1001,7 +1007,8 @@ static int enqueue_evaluation(mbpol_context* ctx, double* forces_dev_out, uint32
         if (!ctx->fork_early) HIP_TRY(hipEventRecord(ctx->ev_fork, st));
         HIP_TRY(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
         forked = true;
-        const int e = short_range(ctx, ctx->side, comp);
+        int e = short_range(ctx, ctx->side, comp);
+        if (!e) e = launch_status();  // errors are kept per thread, and this may be the side enqueuer's
         // recorded also after a failure, so that the join below completes a capture
         HIP_TRY(hipEventRecord(ctx->ev_join, ctx->side));
         return e;
@@ -1034,7 +1041,7 @@ static int enqueue_evaluation(mbpol_context* ctx, double* forces_dev_out, uint32
     if (int e = results_to_host(ctx, st)) return e;
     if (forces_host_out)
         HIP_TRY(hipMemcpyAsync(forces_host_out, fout, sizeof(double) * 3 * s.n, hipMemcpyDeviceToHost, st));
-    return MBPOL_OK;
+    return launch_status();
 }
 
 // the five component energies and their total, from the fixed-point sums read back
