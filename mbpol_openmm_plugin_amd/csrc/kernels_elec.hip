@@ -1475,27 +1475,57 @@ __global__ void k_add_forces_fix(int n, const double* __restrict__ f, u64* __res
 
 // potential of the charges and induced dipoles at arbitrary points
 // (calculateElectrostaticPotentialForParticleGridPoint, :1023-1086): plain
-// Coulomb sum over every site, nearest image under PME.  A wave per point, its lanes
-// over the sites: with a thread per point, 8000 points were 125 waves on 1024 SIMDs
-// and each walked all sites (259 us for 1024 sites, 30 now).
+// Coulomb sum over every site, nearest image under PME.  G lanes take M points; a
+// point's sum is formed in 64 parts (sites p, p + 64, ...), 64 / G of them a lane, which
+// are then added in pairs (p and p + 32, then p + 16, ..., p + 1), the same way for
+// every G and M: a point's potential does not depend on how many points are asked for.
+template <int G, int M>
 __global__ void __launch_bounds__(256) k_potential_at_points(int npts, const double* __restrict__ pts, int n,
                                                              const double* __restrict__ pos, const double* __restrict__ q,
                                                              const double* __restrict__ mu, ElecParams P,
                                                              double* __restrict__ out) {
     critical_path_wave();
-    const int k = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (k >= npts) return;
-    const double x = pts[3 * k], y = pts[3 * k + 1], z = pts[3 * k + 2];
-    double v = 0.0;
-    for (int i = lane; i < n; i += 64) {
-        double dx = pos[3 * i] - x, dy = pos[3 * i + 1] - y, dz = pos[3 * i + 2] - z;
-        min_image(dx, dy, dz, P);
-        const double r2 = dx * dx + dy * dy + dz * dz, r = sqrt(r2);
-        const double rr1 = 1.0 / r, rr3 = rr1 / r2;
-        v += q[i] * rr1 - (mu[3 * i] * dx + mu[3 * i + 1] * dy + mu[3 * i + 2] * dz) * rr3;
+    constexpr int K = 64 / G;
+    const int lane = threadIdx.x % G;
+    const int k0 = (int)((blockIdx.x * blockDim.x + threadIdx.x) / G) * M;
+    if (k0 >= npts) return;
+    double x[M], y[M], z[M], v[M][K];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        const size_t k = min(k0 + m, npts - 1);
+        x[m] = pts[3 * k];
+        y[m] = pts[3 * k + 1];
+        z[m] = pts[3 * k + 2];
+#pragma unroll
+        for (int u = 0; u < K; ++u) v[m][u] = 0.0;
     }
-    v = wave_sum(v);
-    if (lane == 0) out[k] = v * el_electric;
+    for (int base = 0; base < n; base += 64)
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const int i = base + u * G + lane;
+            if (i < n) {
+                const double px = pos[3 * i], py = pos[3 * i + 1], pz = pos[3 * i + 2], qi = q[i];
+                const double mx = mu[3 * i], my = mu[3 * i + 1], mz = mu[3 * i + 2];
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    double dx = px - x[m], dy = py - y[m], dz = pz - z[m];
+                    min_image(dx, dy, dz, P);
+                    const double r2 = dx * dx + dy * dy + dz * dz, r = sqrt(r2);
+                    const double rr1 = 1.0 / r, rr3 = rr1 / r2;
+                    v[m][u] += qi * rr1 - (mx * dx + my * dy + mz * dz) * rr3;
+                }
+            }
+        }
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+#pragma unroll
+        for (int off = K / 2; off > 0; off >>= 1)
+#pragma unroll
+            for (int u = 0; u < off; ++u) v[m][u] += v[m][u + off];
+#pragma unroll
+        for (int off = G / 2; off > 0; off >>= 1) v[m][0] += __shfl_xor(v[m][0], off, G);
+        if (lane == 0 && k0 + m < npts) out[k0 + m] = v[m][0] * el_electric;
+    }
 }
 
 // System multipole moments about the centre of mass (MBPolReferenceElectrostaticsForce.cpp:923-1021),
@@ -1718,7 +1748,21 @@ void launch_energy_finish(hipStream_t s, int nblocks, const double* eblk, u64* e
 }
 void launch_potential_at_points(hipStream_t s, int npts, const double* pts, int n, const double* pos, const double* q,
                                 const double* mu, ElecParams P, double* out) {
-    hipLaunchKernelGGL(k_potential_at_points, nblk(64LL * npts, 256), 256, 0, s, npts, pts, n, pos, q, mu, P, out);
+    // Few points: a wave each.  Many: 16 lanes take four points, whose site loads they share.  A call with its
+    // copies in us, a thread a point / a wave / 16 lanes for 4 points: 256 waters, 8000 points 395 / 169 / 193,
+    // 50,000 398 / 257 / 259, 1,000,000 3650 / 4230 / 3570; 14 waters, 50,000 124 / 127 / 118, 1,000,000
+    // 1300 / 1470 / 1330.  A launch takes 2^26 points at most, below the 2^32 threads it may have.
+    constexpr long long kFew = 32768, kLaunch = 1 << 26;
+    for (long long first = 0; first < npts; first += kLaunch) {
+        const int m = (int)std::min<long long>(npts - first, kLaunch);
+        const double* p = pts + 3 * first;
+        if (npts <= kFew)
+            hipLaunchKernelGGL((k_potential_at_points<64, 1>), nblk(64LL * m, 256), 256, 0, s, m, p, n, pos, q, mu, P,
+                               out + first);
+        else
+            hipLaunchKernelGGL((k_potential_at_points<16, 4>), nblk((m + 3LL) / 4 * 16, 256), 256, 0, s, m, p, n, pos, q,
+                               mu, P, out + first);
+    }
 }
 void launch_system_moments(hipStream_t s, int n, const double* pos, const double* q, const double* mu,
                            const double* mass, double* out) {
