@@ -110,21 +110,20 @@ void launch_offsets_of(hipStream_t s, int n, const int* start, int limit, const 
 // ---- kernels_pip.hip (one object per body order and precision) ----
 // n: the list's capacity (grid size); ndev (optional): its length on the device (the kernels
 // stop there); max_blocks > 0 caps the grid (64-lane blocks), the kernels then stride over the list
-#define MBPOL_PIP_LAUNCHER(name, T)                                                                             \
+#define MBPOL_PIP_LAUNCHER(name, T, ...)                                                                        \
     void name(hipStream_t s, long long n, const long long* ndev, const T* list, const int* idx, const double* pos, \
-              int periodic, d3 box, u64* force, u64* energy, const KEvents& ev = KEvents(), double* eunit = nullptr, \
-              int max_blocks = 0)
+              int periodic, d3 box, u64* force, u64* energy, __VA_ARGS__ const KEvents& ev, double* eunit,       \
+              int max_blocks)
 // 2-body, term by term (the coefficients as instruction literals)
-MBPOL_PIP_LAUNCHER(launch_twobody_f32, int2);
-MBPOL_PIP_LAUNCHER(launch_twobody_f64, int2);
-// the 2-body polynomial through the dimer's relabelling group (pip_orbit_loop.h), FP32 and FP64
-MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f32, int2);
-MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f64, int2);
+MBPOL_PIP_LAUNCHER(launch_twobody_f32, int2, );
+MBPOL_PIP_LAUNCHER(launch_twobody_f64, int2, );
 // FP64, term by term (the coefficients as instruction literals)
-MBPOL_PIP_LAUNCHER(launch_threebody_f64, int);
-// the polynomial through its relabelling group (pip_orbit_loop.h), FP32 and FP64
-MBPOL_PIP_LAUNCHER(launch_threebody_orbit_f32, int);
-MBPOL_PIP_LAUNCHER(launch_threebody_orbit_f64, int);
+MBPOL_PIP_LAUNCHER(launch_threebody_f64, int, );
+// the polynomials through their relabelling groups (pip_orbit_loop.h), FP32 and FP64; cus: compute units of the device
+MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f32, int2, int cus, );
+MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f64, int2, int cus, );
+MBPOL_PIP_LAUNCHER(launch_threebody_orbit_f32, int, int cus, );
+MBPOL_PIP_LAUNCHER(launch_threebody_orbit_f64, int, int cus, );
 #undef MBPOL_PIP_LAUNCHER
 
 }  // namespace mbpol

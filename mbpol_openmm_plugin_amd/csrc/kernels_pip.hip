@@ -709,6 +709,8 @@ __global__ void __launch_bounds__(64) k_threebody(long long nt, const long long*
 //      one wave after the other: the sums do not depend on scheduling;
 //   4. the waves take the points in turn for the chain rule;
 //   5. wave m sums and adds the forces of molecule m, the wave after them the energy.
+// Q follows from the list's length on the device, not from the capacity the host launches
+// by, so that a configuration's results do not depend on those evaluated before it.
 // Steps 2 and 4 are rolled loops over tables of the variables, so that a unit's
 // code outside the passes is short and, for a short list, not fetched in vain.
 //
@@ -762,8 +764,18 @@ __device__ __forceinline__ float rsqrt_pip(float v) { return 1.0f / sqrtf(v); }
 
 constexpr int P = 4;  // waves of a block
 
+// Blocks a unit's passes are spread over: as many as still find a CU each, since
+// only then does every wave have a SIMD to itself, and a short list takes as long
+// as one wave's passes.
+__host__ __device__ constexpr int unit_parts(long long units, int cus) {
+    for (int q : {6, 3, 2})
+        if (kPassAll % (P * q) == 0 && units * q <= cus) return q;
+    return 1;
+}
+constexpr int kMostParts = unit_parts(1, 1 << 20);
+
 __global__ void __launch_bounds__(64 * P) __attribute__((amdgpu_waves_per_eu(2)))
-k_pip_split(int parts, long long nu, const long long* __restrict__ ndev, const Unit* __restrict__ list,
+k_pip_split(int cus, long long nu, const long long* __restrict__ ndev, const Unit* __restrict__ list,
             const int* __restrict__ idx, const double* __restrict__ pos, int periodic, d3 box,
             u64* __restrict__ force, u64* __restrict__ energy, double* __restrict__ eunit) {
     constexpr int N = kVars;
@@ -775,8 +787,12 @@ k_pip_split(int parts, long long nu, const long long* __restrict__ ndev, const U
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     PIP_CONST_PTR(PipTables) tab = (PIP_CONST_PTR(PipTables))&pip_tables;
     if (ndev) nu = min(nu, *ndev);
+    int parts = eunit ? 1 : unit_parts((nu + 63) / 64, cus);  // a unit's energy is written whole by one block
+    PIP_OPAQUE_PTR(parts);  // one copy of the code for every value
     const int part = blockIdx.x % parts, npass = kPassAll / (P * parts), k0 = (part * P + wave) * npass;
-    for (long long t0 = (long long)(blockIdx.x / parts) * 64; t0 < nu; t0 += (long long)(gridDim.x / parts) * 64) {
+    // with several blocks a unit the grid has one for every part of every unit (split_grid)
+    const long long stride = parts > 1 ? nu : (long long)gridDim.x * 64;
+    for (long long t0 = (long long)(blockIdx.x / parts) * 64; t0 < nu; t0 += stride) {
         const long long t = t0 + lane;
         if (wave == 0) {
             bool on = false;
@@ -879,34 +895,22 @@ static inline int grid(long long n, int max_waves, int waves) {
     return (int)(max_waves > 0 && b > cap ? cap : b);
 }
 #if PIP_ORBIT
-// Blocks a unit's passes are spread over: as many as still find a CU each, since
-// only then does every wave have a SIMD to itself, and a short list takes as long
-// as one wave's passes.  Not with unit energies, which one block writes whole.
-static int unit_parts(long long n, bool eunit) {
-    static const int cus = [] {
-        int d = 0, c = 0;
-        const bool ok = hipGetDevice(&d) == hipSuccess &&
-                        hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, d) == hipSuccess;
-        return ok && c > 0 ? c : 256;
-    }();
-    const long long units = (n + 63) / 64;
-    for (int q : {6, 3, 2})
-        if (!eunit && kPassAll % (P * q) == 0 && units * q <= cus) return q;
-    return 1;
+// One block per 64 units at most max_waves / P of them, but a block for every part of every unit of any list
+// that unit_parts would split (units * parts <= cus of them).
+static inline int split_grid(long long n, int max_waves, int cus) {
+    return std::max(grid(n, max_waves, P), (int)std::min<long long>((n + 63) / 64 * kMostParts, cus));
 }
-#define PIP_LAUNCH(kern, n, s, ...)                                                                         \
-    do {                                                                                                    \
-        const int parts = unit_parts(n, eunit != nullptr);                                                  \
-        MBPOL_LAUNCH(ev, k_pip_split, parts > 1 ? parts * grid(n, 0, P) : grid(n, max_blocks, P), 64 * P, 0, \
-                     s, parts, __VA_ARGS__);                                                                \
-    } while (0)
+#define PIP_CUS int cus,
+#define PIP_LAUNCH(kern, n, s, ...) \
+    MBPOL_LAUNCH(ev, k_pip_split, split_grid(n, max_blocks, cus), 64 * P, 0, s, cus, __VA_ARGS__)
 #else
+#define PIP_CUS
 #define PIP_LAUNCH(kern, n, s, ...) MBPOL_LAUNCH(ev, kern, grid(n, max_blocks, 1), 64, 0, s, __VA_ARGS__)
 #endif
 #if PIP_BODY == 2
 void PIP_CAT(launch_twobody_, PIP_SUFFIX)(hipStream_t s, long long npairs, const long long* ndev, const int2* pairs,
                                           const int* idx, const double* pos, int periodic, d3 box, u64* force,
-                                          u64* energy, const KEvents& ev, double* eunit, int max_blocks) {
+                                          u64* energy, PIP_CUS const KEvents& ev, double* eunit, int max_blocks) {
 #if !PIP_ORBIT
     box = d3{box.x * 10., box.y * 10., box.z * 10.};
 #endif
@@ -917,7 +921,7 @@ void PIP_CAT(launch_twobody_, PIP_SUFFIX)(hipStream_t s, long long npairs, const
 #else
 void PIP_CAT(launch_threebody_, PIP_SUFFIX)(hipStream_t s, long long ntrip, const long long* ndev, const int* trip,
                                             const int* idx, const double* pos, int periodic, d3 box, u64* force,
-                                            u64* energy, const KEvents& ev, double* eunit, int max_blocks) {
+                                            u64* energy, PIP_CUS const KEvents& ev, double* eunit, int max_blocks) {
     if (ntrip > 0)
         PIP_LAUNCH(k_threebody, ntrip, s, ntrip, ndev, trip, idx, pos, periodic, box,
                      force, energy, eunit);

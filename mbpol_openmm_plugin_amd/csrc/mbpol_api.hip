@@ -902,10 +902,14 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
             const KEvents ev = timer_kernel(ctx, T_TWOBODY);
             const long long* nd = ctx->dimer_off.as<long long>() + (int)s.tb_idx.size() / 3;  // list length (device)
             // the polynomial through the dimer's relabelling group, or term by term (MBPOL_HIP_2B_KERNEL=terms)
-            auto launch2 = dp ? (ctx->pip2_kernel == 1 ? launch_twobody_f64 : launch_twobody_orbit_f64)
-                              : (ctx->pip2_kernel == 1 ? launch_twobody_f32 : launch_twobody_orbit_f32);
-            launch2(sr, ctx->dimer_cap, nd, ctx->dimers.as<int2>(), ctx->tb_idx.as<int>(), pos, per, box, F, E + 1, ev,
-                    eu2, ctx->pip_blocks);
+            const int2* dl = ctx->dimers.as<int2>();
+            const int* ti = ctx->tb_idx.as<int>();
+            if (ctx->pip2_kernel == 1)
+                (dp ? launch_twobody_f64 : launch_twobody_f32)(sr, ctx->dimer_cap, nd, dl, ti, pos, per, box, F, E + 1, ev,
+                                                               eu2, ctx->pip_blocks);
+            else
+                (dp ? launch_twobody_orbit_f64 : launch_twobody_orbit_f32)(sr, ctx->dimer_cap, nd, dl, ti, pos, per, box, F,
+                                                                           E + 1, ctx->cus, ev, eu2, ctx->pip_blocks);
             timer_kernel_done(ctx, T_TWOBODY, ev);
             // dimers are listed by their first molecule, so a group's dimers are consecutive
             if (G)
@@ -923,12 +927,11 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
             const int* tr = ctx->trips.as<int>();
             const int* ti = ctx->th_idx.as<int>();
             const int cap = ctx->pip3_blocks;
-            if (!dp)
-                launch_threebody_orbit_f32(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2, ev, eu3, cap);
-            else if (ctx->pip3_kernel == 1)
+            if (dp && ctx->pip3_kernel == 1)
                 launch_threebody_f64(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2, ev, eu3, cap);
             else
-                launch_threebody_orbit_f64(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2, ev, eu3, cap);
+                (dp ? launch_threebody_orbit_f64 : launch_threebody_orbit_f32)(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2,
+                                                                               ctx->cus, ev, eu3, cap);
             timer_kernel_done(ctx, T_THREEBODY, ev);
             if (G) {
                 const int n3 = (int)s.th_idx.size() / 3;
