@@ -119,11 +119,20 @@ MBPOL_PIP_LAUNCHER(launch_twobody_f32, int2, );
 MBPOL_PIP_LAUNCHER(launch_twobody_f64, int2, );
 // FP64, term by term (the coefficients as instruction literals)
 MBPOL_PIP_LAUNCHER(launch_threebody_f64, int, );
-// the polynomials through their relabelling groups (pip_orbit_loop.h), FP32 and FP64; cus: compute units of the device
-MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f32, int2, int cus, );
-MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f64, int2, int cus, );
-MBPOL_PIP_LAUNCHER(launch_threebody_orbit_f32, int, int cus, );
-MBPOL_PIP_LAUNCHER(launch_threebody_orbit_f64, int, int cus, );
+// What the blocks that share a unit leave for the kernel that joins them (short lists): `slots` shares of
+// kPipRows x 64 numbers and as many rows of points.  One per context: its 2- and 3-body kernels run one after
+// the other.
+constexpr int kPipRows = 31;
+struct PipScratch {
+    void* shares;
+    double* points;
+    int slots;  // compute units of the device
+};
+// the polynomials through their relabelling groups (pip_orbit_loop.h), FP32 and FP64
+MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f32, int2, const PipScratch& scratch, );
+MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f64, int2, const PipScratch& scratch, );
+MBPOL_PIP_LAUNCHER(launch_threebody_orbit_f32, int, const PipScratch& scratch, );
+MBPOL_PIP_LAUNCHER(launch_threebody_orbit_f64, int, const PipScratch& scratch, );
 #undef MBPOL_PIP_LAUNCHER
 
 }  // namespace mbpol

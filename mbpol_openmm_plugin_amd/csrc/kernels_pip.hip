@@ -709,8 +709,13 @@ __global__ void __launch_bounds__(64) k_threebody(long long nt, const long long*
 //      one wave after the other: the sums do not depend on scheduling;
 //   4. the waves take the points in turn for the chain rule;
 //   5. wave m sums and adds the forces of molecule m, the wave after them the energy.
-// Q follows from the list's length on the device, not from the capacity the host launches
-// by, so that a configuration's results do not depend on those evaluated before it.
+// With Q > 1 the blocks write their shares of the points' gradient and of the energy to
+// memory instead, and k_pip_join adds a unit's shares in their order before step 5: a
+// unit's sums are formed in floating point and rounded to fixed point once.  (The last of
+// the blocks doing so in this kernel, behind fences, took as long and put registers of
+// the passes into scratch.)  Q follows from the list's length on the device, not from the
+// capacity the host launches by, so that a configuration's results do not depend on those
+// evaluated before it.
 // Steps 2 and 4 are rolled loops over tables of the variables, so that a unit's
 // code outside the passes is short and, for a short list, not fetched in vain.
 //
@@ -720,22 +725,21 @@ __global__ void __launch_bounds__(64) k_threebody(long long nt, const long long*
 // allow; a short one lasts as long as one wave's share of the passes, so it is cut
 // finer until the waves would meet on a SIMD again (8 waves in one block on one CU
 // gained nothing over 4).  One wave per unit through all passes (2-body: term by
-// term) took, against this: 101 trimers 207 / 42 us, 13,641 238 / 101, 139,535
-// 566 / 450; 91 dimers 93 / 32, 4612 93 / 47, 42,250 105 / 83.
+// term) took 207 us for 101 trimers, 238 for 13,641, 566 for 139,535; 93 for 91 dimers,
+// 93 for 4612, 105 for 42,250.  Both kernels here: 101 trimers 38-51 (from one call to
+// the next alone, or beside the other terms), 776 41, 9204 88, 134,272 638; 91 dimers
+// 40, 2016 44, 42,250 86 -- the join is 4-6 of each, and an idle launch for long lists.
 // ---------------------------------------------------------------------------
 #if PIP_BODY == 2
 constexpr int kPoints = 10, kVars = 31, kMols = 2, kPassAll = pip2b_npass;
 typedef Var2 Var;
 typedef int2 Unit;
 __host__ __device__ constexpr Var var_of(int n) { return var2(n); }
-// points of molecule m: its atoms, then its extra points
-__device__ __forceinline__ int molecule_of(const Unit* list, long long t, int m) { return m ? list[t].y : list[t].x; }
 #else
 constexpr int kPoints = 9, kVars = 36, kMols = 3, kPassAll = pip3b_npass;
 typedef Var3 Var;
 typedef int Unit;
 __host__ __device__ constexpr Var var_of(int n) { return var3(n); }
-__device__ __forceinline__ int molecule_of(const Unit* list, long long t, int m) { return list[3 * t + m]; }
 #endif
 // the variables, and for every point the variables it enters with the point at the other end
 struct Partner {
@@ -763,19 +767,21 @@ __device__ __forceinline__ double rsqrt_pip(double v) { return rsqrt(v); }
 __device__ __forceinline__ float rsqrt_pip(float v) { return 1.0f / sqrtf(v); }
 
 constexpr int P = 4;  // waves of a block
+constexpr int kXYZ = 3 * kPoints;
+static_assert(kXYZ + 1 <= kPipRows, "the rows of a share: the points' gradient, the energy");
 
 // Blocks a unit's passes are spread over: as many as still find a CU each, since
 // only then does every wave have a SIMD to itself, and a short list takes as long
 // as one wave's passes.
-__host__ __device__ constexpr int unit_parts(long long units, int cus) {
+__host__ __device__ constexpr int unit_parts(long long units, int slots) {
     for (int q : {6, 3, 2})
-        if (kPassAll % (P * q) == 0 && units * q <= cus) return q;
+        if (kPassAll % (P * q) == 0 && units * q <= slots) return q;
     return 1;
 }
 constexpr int kMostParts = unit_parts(1, 1 << 20);
 
 __global__ void __launch_bounds__(64 * P) __attribute__((amdgpu_waves_per_eu(2)))
-k_pip_split(int cus, long long nu, const long long* __restrict__ ndev, const Unit* __restrict__ list,
+k_pip_split(PipScratch scratch, long long nu, const long long* __restrict__ ndev, const Unit* __restrict__ list,
             const int* __restrict__ idx, const double* __restrict__ pos, int periodic, d3 box,
             u64* __restrict__ force, u64* __restrict__ energy, double* __restrict__ eunit) {
     constexpr int N = kVars;
@@ -787,12 +793,10 @@ k_pip_split(int cus, long long nu, const long long* __restrict__ ndev, const Uni
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     PIP_CONST_PTR(PipTables) tab = (PIP_CONST_PTR(PipTables))&pip_tables;
     if (ndev) nu = min(nu, *ndev);
-    int parts = eunit ? 1 : unit_parts((nu + 63) / 64, cus);  // a unit's energy is written whole by one block
+    int parts = unit_parts((nu + 63) / 64, scratch.slots);
     PIP_OPAQUE_PTR(parts);  // one copy of the code for every value
     const int part = blockIdx.x % parts, npass = kPassAll / (P * parts), k0 = (part * P + wave) * npass;
-    // with several blocks a unit the grid has one for every part of every unit (split_grid)
-    const long long stride = parts > 1 ? nu : (long long)gridDim.x * 64;
-    for (long long t0 = (long long)(blockIdx.x / parts) * 64; t0 < nu; t0 += stride) {
+    for (long long t0 = (long long)(blockIdx.x / parts) * 64; t0 < nu; t0 += (long long)gridDim.x * 64) {
         const long long t = t0 + lane;
         if (wave == 0) {
             bool on = false;
@@ -872,6 +876,24 @@ k_pip_split(int cus, long long nu, const long long* __restrict__ ndev, const Uni
             fs[3 * p + 2][lane] = F.z;
         }
         __syncthreads();
+        if (parts > 1) {  // the block's only unit: the grid has a block for every part of every unit
+            int ln = lane;  // opaque copies: no address of this part is kept in registers through the passes
+            asm volatile("" : "+v"(ln));
+            real* share = static_cast<real*>(scratch.shares) + (size_t)blockIdx.x * (kPipRows * 64);
+            double* points = scratch.points + (size_t)(blockIdx.x / parts) * (kPipRows * 64);
+            PIP_OPAQUE_PTR(share);
+            PIP_OPAQUE_PTR(points);
+#pragma nounroll
+            for (int r = wave; r < kXYZ; r += P) {
+                share[r * 64 + ln] = fs[r][ln];
+                if (part == 0) points[r * 64 + ln] = rs[r][ln];
+            }
+            if (wave == 0) {
+                share[kXYZ * 64 + ln] = es[0][ln] + es[1][ln] + es[2][ln] + es[3][ln];
+                if (part == 0) points[kXYZ * 64 + ln] = on ? 1.0 : 0.0;
+            }
+            return;
+        }
         if (wave <= kMols) {
             real E = es[0][lane];
 #pragma unroll
@@ -880,6 +902,47 @@ k_pip_split(int cus, long long nu, const long long* __restrict__ ndev, const Uni
         }
         __syncthreads();  // the LDS arrays are written again
     }
+}
+
+// step 5 of the units whose passes were spread over several blocks, a block per unit
+__global__ void __launch_bounds__(64 * P)
+k_pip_join(PipScratch scratch, long long nu, const long long* __restrict__ ndev, const Unit* __restrict__ list,
+           const int* __restrict__ idx, u64* __restrict__ force, u64* __restrict__ energy,
+           double* __restrict__ eunit) {
+    __shared__ double rs[kXYZ][64], ons[64];
+    __shared__ real fs[kXYZ][64], es[64];
+    if (ndev) nu = min(nu, *ndev);
+    const int unit = blockIdx.x, parts = unit_parts((nu + 63) / 64, scratch.slots);
+    const long long t = (long long)unit * 64 + (threadIdx.x & 63);
+    if (parts == 1 || (long long)unit * 64 >= nu) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int R = (kXYZ + 1 + P - 1) / P;  // rows of a wave
+    const real* shares = static_cast<const real*>(scratch.shares) + (size_t)unit * parts * (kPipRows * 64) + lane;
+    const double* points = scratch.points + (size_t)unit * (kPipRows * 64) + lane;
+    real v[kMostParts][R];
+    double x[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {  // every load in flight at once (past the last part or row: that one again)
+        const int r = min(wave + P * i, kXYZ);
+        x[i] = points[r * 64];
+#pragma unroll
+        for (int p = 0; p < kMostParts; ++p) v[p][i] = shares[(min(p, parts - 1) * kPipRows + r) * 64];
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int r = wave + P * i;
+        real sum = v[0][i];
+#pragma unroll
+        for (int p = 1; p < kMostParts; ++p)
+            if (p < parts) sum += v[p][i];
+        if (r <= kXYZ) {
+            (r < kXYZ ? rs[r] : ons)[lane] = x[i];
+            (r < kXYZ ? fs[r] : es)[lane] = sum;
+        }
+    }
+    __syncthreads();
+    if (wave <= kMols)
+        unit_end(wave, ons[lane] != 0.0, t, t < nu, (double)es[lane], rs, fs, list, idx, force, energy, eunit, lane);
 }
 #endif
 
@@ -896,21 +959,33 @@ static inline int grid(long long n, int max_waves, int waves) {
 }
 #if PIP_ORBIT
 // One block per 64 units at most max_waves / P of them, but a block for every part of every unit of any list
-// that unit_parts would split (units * parts <= cus of them).
-static inline int split_grid(long long n, int max_waves, int cus) {
-    return std::max(grid(n, max_waves, P), (int)std::min<long long>((n + 63) / 64 * kMostParts, cus));
+// that unit_parts would split (units * parts <= slots of them); and those lists' second kernel.
+static inline int split_grid(long long n, int max_waves, int slots) {
+    return std::max(grid(n, max_waves, P), (int)std::min<long long>((n + 63) / 64 * kMostParts, slots));
 }
-#define PIP_CUS int cus,
-#define PIP_LAUNCH(kern, n, s, ...) \
-    MBPOL_LAUNCH(ev, k_pip_split, split_grid(n, max_blocks, cus), 64 * P, 0, s, cus, __VA_ARGS__)
+static inline int join_grid(long long n, int slots) { return (int)std::min<long long>((n + 63) / 64, slots / 2); }
+#define PIP_SCRATCH const PipScratch &scratch,
+#define PIP_LAUNCH(kern, n, s, np, ndev, list, idx, ...)                                                             \
+    do {                                                                                                             \
+        const int blocks = split_grid(n, max_blocks, scratch.slots), joins = join_grid(n, scratch.slots);            \
+        if (ev.start) { /* the span of both */                                                                       \
+            hipExtLaunchKernelGGL(k_pip_split, blocks, 64 * P, 0, s, ev.start, nullptr, 0, scratch, np, ndev, list,  \
+                                  idx, __VA_ARGS__);                                                                 \
+            hipExtLaunchKernelGGL(k_pip_join, joins, 64 * P, 0, s, nullptr, ev.stop, 0, scratch, np, ndev, list,     \
+                                  idx, force, energy, eunit);                                                        \
+        } else {                                                                                                     \
+            hipLaunchKernelGGL(k_pip_split, blocks, 64 * P, 0, s, scratch, np, ndev, list, idx, __VA_ARGS__);        \
+            hipLaunchKernelGGL(k_pip_join, joins, 64 * P, 0, s, scratch, np, ndev, list, idx, force, energy, eunit); \
+        }                                                                                                            \
+    } while (0)
 #else
-#define PIP_CUS
+#define PIP_SCRATCH
 #define PIP_LAUNCH(kern, n, s, ...) MBPOL_LAUNCH(ev, kern, grid(n, max_blocks, 1), 64, 0, s, __VA_ARGS__)
 #endif
 #if PIP_BODY == 2
 void PIP_CAT(launch_twobody_, PIP_SUFFIX)(hipStream_t s, long long npairs, const long long* ndev, const int2* pairs,
                                           const int* idx, const double* pos, int periodic, d3 box, u64* force,
-                                          u64* energy, PIP_CUS const KEvents& ev, double* eunit, int max_blocks) {
+                                          u64* energy, PIP_SCRATCH const KEvents& ev, double* eunit, int max_blocks) {
 #if !PIP_ORBIT
     box = d3{box.x * 10., box.y * 10., box.z * 10.};
 #endif
@@ -921,7 +996,7 @@ void PIP_CAT(launch_twobody_, PIP_SUFFIX)(hipStream_t s, long long npairs, const
 #else
 void PIP_CAT(launch_threebody_, PIP_SUFFIX)(hipStream_t s, long long ntrip, const long long* ndev, const int* trip,
                                             const int* idx, const double* pos, int periodic, d3 box, u64* force,
-                                            u64* energy, PIP_CUS const KEvents& ev, double* eunit, int max_blocks) {
+                                            u64* energy, PIP_SCRATCH const KEvents& ev, double* eunit, int max_blocks) {
     if (ntrip > 0)
         PIP_LAUNCH(k_threebody, ntrip, s, ntrip, ndev, trip, idx, pos, periodic, box,
                      force, energy, eunit);

@@ -608,6 +608,11 @@ int mbpol_context_create(const mbpol_system* sys, int32_t precision, int32_t dev
         if (ctx->lo_count.ensure(sizeof(int) * (n3 + 1)) || ctx->lo_start.ensure(sizeof(int) * (n3 + 1)))
             return fail(set_error(MBPOL_ERR_HIP, "device allocation failed"));
     }
+    if (n2 > 0 || n3 > 0) {
+        const size_t bytes = sizeof(double) * 64 * kPipRows * ctx->cus;
+        if (ctx->pip_shares.ensure(bytes) || ctx->pip_points.ensure(bytes))
+            return fail(set_error(MBPOL_ERR_HIP, "device allocation failed"));
+    }
     apply_list_groups(ctx);
     if (sys->ne > 0) {
         if (int e = elec_create(ctx)) return fail(e);
@@ -896,6 +901,7 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
     // terms cancel to ~1e-3 of their magnitudes, so FP32 evaluation loses three
     // digits of the 2- and 3-body energies.
     const bool dp = ctx->precision != MBPOL_PRECISION_SINGLE_PIP;
+    const PipScratch scratch{ctx->pip_shares.p, ctx->pip_points.as<double>(), ctx->cus};
     auto run2 = [&]() -> int {
         if (do2) {
             const int per = s.tb_method == MBPOL_CUTOFF_PERIODIC;
@@ -909,7 +915,7 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
                                                                eu2, ctx->pip_blocks);
             else
                 (dp ? launch_twobody_orbit_f64 : launch_twobody_orbit_f32)(sr, ctx->dimer_cap, nd, dl, ti, pos, per, box, F,
-                                                                           E + 1, ctx->cus, ev, eu2, ctx->pip_blocks);
+                                                                           E + 1, scratch, ev, eu2, ctx->pip_blocks);
             timer_kernel_done(ctx, T_TWOBODY, ev);
             // dimers are listed by their first molecule, so a group's dimers are consecutive
             if (G)
@@ -931,7 +937,7 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
                 launch_threebody_f64(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2, ev, eu3, cap);
             else
                 (dp ? launch_threebody_orbit_f64 : launch_threebody_orbit_f32)(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2,
-                                                                               ctx->cus, ev, eu3, cap);
+                                                                               scratch, ev, eu3, cap);
             timer_kernel_done(ctx, T_THREEBODY, ev);
             if (G) {
                 const int n3 = (int)s.th_idx.size() / 3;
