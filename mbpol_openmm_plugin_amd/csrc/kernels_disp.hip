@@ -138,10 +138,10 @@ __global__ void __launch_bounds__(64) k_disp(DispGeom g, const int* __restrict__
                 offer(valid, make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], (double)(mol[j] * 16 + type[j])));
             }
         } else {
-            // Cells of half the cutoff, two each way (125 of them), when the box holds five of them per
-            // axis, else of the cutoff, one each way: 11.4 against 19.7 nm^3 of candidates at 0.9 nm, and
-            // 15 atoms a cell instead of 120 for the counters' atomics and the sort.  15,000 atoms: pair
-            // kernel 91 -> 77 us, cell counts 23 -> 4.4, fill 23 -> 5.7, sort 20 -> 4.2.
+            // Cells of half the cutoff, two each way (125 of them), or of the cutoff, one each way (disp_set_box):
+            // 11.4 against 19.7 nm^3 of candidates at 0.9 nm, and in water 15 atoms a cell instead of 120 for the
+            // counters' atomics and the sort.  15,000 atoms: pair kernel 91 -> 77 us, cell counts 23 -> 4.4, fill
+            // 23 -> 5.7, sort 20 -> 4.2.
             // The cells along z of a column (X, Y) are consecutive in the cell order: one or two member
             // ranges a column, one per lane, laid end to end and taken 64 members at a time.
             const int c = cell_of[a], reach = g.reach, side = 2 * reach + 1;

@@ -43,3 +43,29 @@ def test_dispersion_matches_oracle(mb, oracle, box, lattice, slab):
     print(len(waters), st.getPotentialEnergy(), E['dispersion'], 'force rel rms %.2g' % err, flush=True)
     assert abs(st.getPotentialEnergy() - E['dispersion']) <= 1e-9 * abs(E['dispersion'])
     assert err <= 1e-8
+
+
+@pytest.mark.parametrize('edge', [
+    2.8,    # 6^3 cells of half the cutoff, three atoms each: taken
+    3.2,    # 7^3: cells of the cutoff
+    46.5,
+    650.0,  # half cells would be more than an int holds
+])
+def test_few_waters_in_a_large_box(mb, oracle, edge):
+    rng = np.random.default_rng(9)
+    # a droplet across a corner of the box
+    site = np.stack(np.meshgrid(*(np.arange(6),) * 3, indexing='ij'), axis=-1).reshape(-1, 3)
+    oxygen = (site - 2.5) * 0.31 + rng.uniform(-0.01, 0.01, (len(site), 3))
+    h = np.array([[0.0, 0.0, 0.0], [0.0757, 0.0586, 0.0], [-0.0757, 0.0586, 0.0]])
+    waters = oxygen[:, None, :] + h
+    waters += np.where(waters[:, :1] < 0, edge, 0.0)
+    sysm = mb.forcefield.create_system(len(waters), nonbonded_method='PME', box=edge, components=8)
+    pos = mb.forcefield.water_positions_with_m(waters)
+    ctx = mb.Context(sysm, precision='double')
+    ctx.setPositions(pos)
+    st = ctx.getState(components=8)
+    E, F = oracle.evaluate_system(sysm, pos, components=8)
+    err = np.sqrt(np.mean((st.getForces() - F) ** 2) / np.mean(F ** 2))
+    print(edge, st.getPotentialEnergy(), E['dispersion'], 'force rel rms %.2g' % err, flush=True)
+    assert abs(st.getPotentialEnergy() - E['dispersion']) <= 1e-9 * abs(E['dispersion'])
+    assert err <= 1e-8
