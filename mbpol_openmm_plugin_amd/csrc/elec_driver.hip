@@ -492,6 +492,7 @@ int elec_create(mbpol_context* ctx) {
             return set_error(MBPOL_ERR_INVALID_ARGUMENT, "PME grid %d x %d x %d is too large", grid[0], grid[1], grid[2]);
         for (DevBuf* b : {&E->rowcount, &E->rowstart, &E->rowfill}) HIP_TRY(b->ensure(sizeof(int) * (rows2 + 1)));
         if (lds) {
+            HIP_TRY(dft_allow_lds());
             for (int d = 0; d < 3; ++d) {
                 const int m = grid[d];
                 std::vector<double2> tw(m);

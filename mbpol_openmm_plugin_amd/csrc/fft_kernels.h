@@ -68,6 +68,8 @@ void launch_fft_z_c2r(hipStream_t s, const PmeFft& F, const double2* H, double* 
                       const int* stop = nullptr);
 // the same passes as dense products on the FP64 matrix cores, for lengths up to kDftMaxLength (kernels_dft.hip)
 constexpr int kDftMaxLength = 512;
+// lets their kernels use more than 64 KB of LDS on the current device: once before their launches
+hipError_t dft_allow_lds();
 void launch_dft_z_r2c(hipStream_t s, const PmeFft& F, const double* real, double2* H, const KEvents& ev,
                       const int* stop);
 void launch_dft_y(hipStream_t s, const PmeFft& F, double2* H, int inverse, const KEvents& ev, const int* stop);

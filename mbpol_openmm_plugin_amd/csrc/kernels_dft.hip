@@ -532,27 +532,31 @@ static size_t roots_bytes(const FftAxis& a, int f) { return sizeof(double2) * (s
 static size_t columns_bytes(const FftAxis& a) { return sizeof(double) * kCol * (size_t)(a.n + 1); }
 static size_t z_bytes(const FftAxis& a) { return roots_bytes(a, 1) + sizeof(double) * kColPad * (size_t)(a.n + 1); }
 
-// one kernel with its dynamic LDS, which beyond 64 KB a kernel has to be allowed first
-#define MBPOL_DFT_LAUNCH1(kern, grid, threads_, bytes, ...)                                                 \
-    do {                                                                                                    \
-        if ((bytes) > 64 * 1024)                                                                            \
-            (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
-        MBPOL_LAUNCH(ev, kern, grid, threads_, bytes, __VA_ARGS__);                                         \
-    } while (0)
+hipError_t dft_allow_lds() {
+    for (const void* kern : {(const void*)k_dft_z_r2c, (const void*)k_spread_dft_z_r2c<true>,
+                             (const void*)k_spread_dft_z_r2c<false>, (const void*)k_dft_z_c2r, (const void*)k_dft_y<1>,
+                             (const void*)k_dft_y<2>, (const void*)k_dft_y<3>, (const void*)k_dft_y<4>,
+                             (const void*)k_dft_x_conv<1>, (const void*)k_dft_x_conv<2>, (const void*)k_dft_x_conv<3>,
+                             (const void*)k_dft_x_conv<4>}) {
+        const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
 
 void launch_dft_z_r2c(hipStream_t s, const PmeFft& F, const double* real, double2* H, const KEvents& ev,
                       const int* stop) {
     const int nl = F.ax[0].n * F.ax[1].n;
-    MBPOL_DFT_LAUNCH1(k_dft_z_r2c, nblk(nl, kCol), threads(F.ax[2], 1), z_bytes(F.ax[2]), s, real, H, nl, F.ax[2], F.khp,
+    MBPOL_LAUNCH(ev, k_dft_z_r2c, nblk(nl, kCol), threads(F.ax[2], 1), z_bytes(F.ax[2]), s, real, H, nl, F.ax[2], F.khp,
                  stop);
 }
 void launch_spread_dft_z_r2c(hipStream_t s, const PmeFft& F, const LineTable& T, bool charges, const double* w,
                              double2* H, const KEvents& ev, const int* stop) {
     const int blocks = nblk(T.nlines, kCol), nt = threads(F.ax[2], 1);
     if (charges)
-        MBPOL_DFT_LAUNCH1(k_spread_dft_z_r2c<true>, blocks, nt, z_bytes(F.ax[2]), s, T, w, H, F.ax[2], F.khp, stop);
+        MBPOL_LAUNCH(ev, k_spread_dft_z_r2c<true>, blocks, nt, z_bytes(F.ax[2]), s, T, w, H, F.ax[2], F.khp, stop);
     else
-        MBPOL_DFT_LAUNCH1(k_spread_dft_z_r2c<false>, blocks, nt, z_bytes(F.ax[2]), s, T, w, H, F.ax[2], F.khp, stop);
+        MBPOL_LAUNCH(ev, k_spread_dft_z_r2c<false>, blocks, nt, z_bytes(F.ax[2]), s, T, w, H, F.ax[2], F.khp, stop);
 }
 void launch_spread_lines(hipStream_t s, const LineTable& T, bool charges, const double* w, double* real,
                          const KEvents& ev, const int* stop) {
@@ -566,11 +570,10 @@ void launch_spread_lines(hipStream_t s, const LineTable& T, bool charges, const 
 // the front radix as a template argument
 #define MBPOL_DFT_LAUNCH(kern, f, ...)                             \
     switch (f) {                                                   \
-        case 2: MBPOL_DFT_LAUNCH1(kern<2>, __VA_ARGS__); break;    \
-        case 3: MBPOL_DFT_LAUNCH1(kern<3>, __VA_ARGS__); break;    \
-        case 4: MBPOL_DFT_LAUNCH1(kern<4>, __VA_ARGS__); break;    \
-        case 5: MBPOL_DFT_LAUNCH1(kern<5>, __VA_ARGS__); break;    \
-        default: MBPOL_DFT_LAUNCH1(kern<1>, __VA_ARGS__); break;   \
+        case 2: MBPOL_LAUNCH(ev, kern<2>, __VA_ARGS__); break;     \
+        case 3: MBPOL_LAUNCH(ev, kern<3>, __VA_ARGS__); break;     \
+        case 4: MBPOL_LAUNCH(ev, kern<4>, __VA_ARGS__); break;     \
+        default: MBPOL_LAUNCH(ev, kern<1>, __VA_ARGS__); break;    \
     }
 void launch_dft_y(hipStream_t s, const PmeFft& F, double2* H, int inverse, const KEvents& ev, const int* stop) {
     const FftAxis& a = F.ax[1];
@@ -590,9 +593,8 @@ void launch_dft_z_c2r(hipStream_t s, const PmeFft& F, const double2* H, double* 
                       const int* stop) {
     const int nl = F.ax[0].n * F.ax[1].n;
     const FftAxis& a = F.ax[2];
-    MBPOL_DFT_LAUNCH1(k_dft_z_c2r, nblk(nl, kCol), threads(a, 1),
+    MBPOL_LAUNCH(ev, k_dft_z_c2r, nblk(nl, kCol), threads(a, 1),
                  roots_bytes(a, 1) + 2 * sizeof(double) * kColPad * (size_t)(a.n / 2 + 1), s, H, real, nl, a, F.khp, stop);
 }
-#undef MBPOL_DFT_LAUNCH1
 
 }  // namespace mbpol
