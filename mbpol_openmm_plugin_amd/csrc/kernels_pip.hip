@@ -50,9 +50,9 @@ __device__ __forceinline__ d3 image_near(const d3& ref, const d3& p, const d3& L
               p.z + L.z * floor((ref.z - p.z) * iL.z + 0.5)};
 }
 
+#if !PIP_ORBIT
 __device__ __forceinline__ vr rel(const d3& p, const d3& o) { return vr((real)(p.x - o.x), (real)(p.y - o.y), (real)(p.z - o.z)); }
-
-#if PIP_ORBIT
+#else
 // Forces of one molecule {idx[3 mol ..]} added by the lane that holds its run's sums.
 __device__ __forceinline__ void add_molecule(u64* __restrict__ force, const int* __restrict__ idx, long long mol,
                                              bool last, const u64 (&f)[9]) {
@@ -141,6 +141,7 @@ __device__ __forceinline__ void extra_grads(const vr& O, const vr& H1, const vr&
     fH2 += gh2;
 }
 
+#if !PIP_ORBIT
 // Geometry of dimer t: atom indices, imaged positions (Angstrom) and, when the
 // O-O distance is inside [2, r2f] Angstrom, the ten points relative to Oa.
 // Returns whether the dimer contributes.
@@ -177,6 +178,7 @@ __device__ __forceinline__ bool dimer_geometry(long long t, const int2* __restri
     extra_points(R[3], R[4], R[5], R[8], R[9]);
     return true;
 }
+#endif
 
 // switch and its derivative (mbpol_2body_constants.cpp:98-111), FP64
 __device__ __forceinline__ void switch2(double rOO, double& sw, double& gsw) {
@@ -443,6 +445,7 @@ __device__ __forceinline__ double switch3(double r, double& g) {  // (:103-120)
     return 1.0;
 }
 
+#if !PIP_ORBIT
 // Geometry of trimer t: atom indices, imaged positions, the three O-O vectors
 // (Angstrom) and, unless an O-O distance is below 2 Angstrom (:160-163), the
 // nine points in Angstrom relative to Oa.  Returns whether the trimer contributes.
@@ -483,6 +486,7 @@ __device__ __forceinline__ bool trimer_geometry(long long t, const int* __restri
     }
     return true;
 }
+#endif
 
 #if PIP_ORBIT
 typedef v3<double> vd;
@@ -726,9 +730,10 @@ __global__ void __launch_bounds__(64) k_threebody(long long nt, const long long*
 // finer until the waves would meet on a SIMD again (8 waves in one block on one CU
 // gained nothing over 4).  One wave per unit through all passes (2-body: term by
 // term) took 207 us for 101 trimers, 238 for 13,641, 566 for 139,535; 93 for 91 dimers,
-// 93 for 4612, 105 for 42,250.  Both kernels here: 101 trimers 38-51 (from one call to
-// the next alone, or beside the other terms), 776 41, 9204 88, 134,272 638; 91 dimers
-// 40, 2016 44, 42,250 86 -- the join is 4-6 of each, and an idle launch for long lists.
+// 93 for 4612, 105 for 42,250.  Both kernels here: 101 trimers 38-51 (beside
+// the other terms, or alone), 776 41, 9204 88, 134,272 638 in a grid of one wave a SIMD;
+// 91 dimers 40, 2016 44, 42,250 86 -- the join is 4-6 of each, and an idle launch for
+// long lists.
 // ---------------------------------------------------------------------------
 #if PIP_BODY == 2
 constexpr int kPoints = 10, kVars = 31, kMols = 2, kPassAll = pip2b_npass;
