@@ -1,4 +1,4 @@
-"""Dense-product grid transforms (FP64 matrix cores) against the library transforms.
+"""Dense-product grid transforms (FP64 matrix cores) and mixed-radix ones against the library transforms.
 
 The same PME electrostatics of the 256-water box through the context's own
 choice of passes and through hipFFT (MBPOL_HIP_PME_FFT=hipfft, which the parity
@@ -55,6 +55,23 @@ def test_dense_passes_match_library_transforms(mb, grid):
     e1, f1, n1 = evaluate(mb, grid, None)
     rel_f = np.sqrt(np.mean((f1 - f0) ** 2) / np.mean(f0 ** 2))
     print(grid, 'energy %.10f vs %.10f' % (e1, e0), 'forces %.2g' % rel_f, 'iterations', n1, n0, flush=True)
+    assert n1 == n0
+    assert abs(e1 - e0) <= 1e-10 * abs(e0)
+    assert rel_f <= 1e-10
+
+
+# smooth lengths: two to six stages, radices 2 to 13, the longest; z above 320 has mixed-radix z passes by default
+RADIX = [(12, 15, 16), (30, 32, 33), (63, 64, 65), (48, 50, 52), (84, 77, 99), (121, 143, 144), (125, 128, 126),
+         (18, 20, 324), (16, 18, 512), (16, 512, 18), (512, 18, 16), (16, 18, 1000)]
+
+
+@pytest.mark.parametrize('mode', ['radix', None])
+@pytest.mark.parametrize('grid', RADIX, ids=lambda g: 'x'.join(map(str, g)))
+def test_mixed_radix_passes_match_library_transforms(mb, grid, mode):
+    e0, f0, n0 = evaluate(mb, grid, 'hipfft')
+    e1, f1, n1 = evaluate(mb, grid, mode)
+    rel_f = np.sqrt(np.mean((f1 - f0) ** 2) / np.mean(f0 ** 2))
+    print(grid, mode, 'energy %.10f vs %.10f' % (e1, e0), 'forces %.2g' % rel_f, 'iterations', n1, n0, flush=True)
     assert n1 == n0
     assert abs(e1 - e0) <= 1e-10 * abs(e0)
     assert rel_f <= 1e-10

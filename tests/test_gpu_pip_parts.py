@@ -1,13 +1,13 @@
 """The 2- and 3-body kernels over list lengths that change their launch: lists of
 one unit of 64 and less, remainders of a unit, and lists whose passes are spread
-over 6, 3, 2 and 1 blocks.  Slabs of the 256-water lattice without a box, against
-the term-by-term kernels (pinned to the oracle by the kernel tests).
+over 6, 3 and 2 blocks and over one.  Slabs of the 256-water lattice without a box
+(6, 3, 2) and of the 4096-water one (1), against the term-by-term kernels (pinned to
+the oracle by the kernel tests).
 
 Tolerance: both kernels evaluate in FP64 and differ in summation order (1e-15 of
 the polynomial's terms, which cancel by about 1e3: 1e-12 of the sums; 1e-10 is
 allowed), and every unit's energy and force component is rounded to 2^-32 before it
-is summed, per block that shares the unit: up to one quantum each way and block
-(6 blocks at most against 1), so 8 quanta per unit.
+is summed, so that each unit may add a quantum of difference; 8 are allowed.
 """
 import os
 
@@ -53,4 +53,19 @@ def test_list_lengths(mb, n):
     for term, m in (('twobody', st['num_dimers']), ('threebody', st['num_trimers'])):
         assert abs(e1[term] - e0[term]) <= 1e-10 * abs(e0[term]) + quanta * m
     # a unit moves 18 or 27 force components
+    assert off <= 1e-10 * norm + quanta * np.sqrt(18 * st['num_dimers'] + 27 * st['num_trimers'])
+
+
+@pytest.mark.parametrize('n', [700, 1500])
+def test_long_lists(mb, n):
+    waters = mb.systems.config2()[0][:n]
+    e0, f0, _ = evaluate(mb, waters, 'terms')
+    e1, f1, st = evaluate(mb, waters, 'orbit')
+    assert 2 * ((st['num_dimers'] + 63) // 64) > 256 or n < 1500  # one block a unit on 256 CUs
+    assert 2 * ((st['num_trimers'] + 63) // 64) > 256
+    off, norm = np.linalg.norm(f1 - f0), np.linalg.norm(f0)
+    print(n, 'waters', st['num_dimers'], st['num_trimers'], 'forces off %.2g of %.2g' % (off, norm), e1, flush=True)
+    quanta = 8 * 2.0 ** -32
+    for term, m in (('twobody', st['num_dimers']), ('threebody', st['num_trimers'])):
+        assert abs(e1[term] - e0[term]) <= 1e-10 * abs(e0[term]) + quanta * m
     assert off <= 1e-10 * norm + quanta * np.sqrt(18 * st['num_dimers'] + 27 * st['num_trimers'])

@@ -1,4 +1,4 @@
-"""Electrostatics neighbour rows (a wave per site over the cell ranges) against brute force.
+"""Electrostatics neighbour rows (a wave for four sites of the cell order, over their cells' ranges) against brute force.
 
 The number of site pairs within the cutoff and of (polarisable, polarisable) pairs, exactly, in boxes
 whose columns cross the boundary on either side, with the fewest cells, with edges of their own per
