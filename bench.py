@@ -44,7 +44,14 @@ FLOPS_PER_DIMER = 31.0e3
 # (FETCH_SIZE x 1.885, WRITE_SIZE x 1.000; the runs are summarised under
 # profiles/); kernels not listed (not counted since they were last changed) report null
 MEASURED_TRAFFIC = {
-    'elec_iterate': 85816165,
+    'threebody': 58490000,
+    'twobody': 18680000,
+    'elec_iterate': 85800000,
+    'spread_fft_z': 28750000,
+    'fft_z_r2c': 35820000,
+    'fft_y': 25660000,
+    'fft_x_conv': 38350000,
+    'fft_z_c2r': 25220000,
 }
 
 
@@ -88,8 +95,11 @@ def kernel_models(stats, grid, nsites, npol):
         # line starts, 25 entries per site (site, first z, 3 FP64 weights), its z spline values and
         # derivatives, dipoles, grid write
         'pme_spread': ('bytes', spread + ngrid * 8, 'hbm', PEAK_HBM_GBS, 'GB/s'),
-        'fft_z_r2c': ('bytes', ngrid * 8 + nhalf * 16, 'hbm', PEAK_HBM_GBS, 'GB/s'),
-        # the spreading fused with the z pass: the same reads, half spectrum write
+        # the charges' z pass, fused with their spreading as the dipoles' (line starts of both halves of the
+        # table, entries, spline values and charges, half spectrum write)
+        'fft_z_r2c': ('bytes', (2 * K0 * K1 + 1) * 4 + nsites * (25 * 32 + 40 + 8) + nhalf * 16, 'hbm', PEAK_HBM_GBS,
+                      'GB/s'),
+        # the dipoles' spreading fused with the z pass: the reads of pme_spread, half spectrum write
         'spread_fft_z': ('bytes', spread + nhalf * 16, 'hbm', PEAK_HBM_GBS, 'GB/s'),
         'fft_y': ('bytes', nhalf * 32, 'hbm', PEAK_HBM_GBS, 'GB/s'),
         'fft_x_conv': ('bytes', nhalf * 40, 'hbm', PEAK_HBM_GBS, 'GB/s'),
