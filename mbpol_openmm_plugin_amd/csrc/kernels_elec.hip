@@ -1751,7 +1751,7 @@ void launch_potential_at_points(hipStream_t s, int npts, const double* pts, int 
     // Few points: a wave each.  Many: 16 lanes take four points, whose site loads they share.  A call with its
     // copies in us, a thread a point / a wave / 16 lanes for 4 points: 256 waters, 8000 points 395 / 169 / 193,
     // 50,000 398 / 257 / 259, 1,000,000 3650 / 4230 / 3570; 14 waters, 50,000 124 / 127 / 118, 1,000,000
-    // 1300 / 1470 / 1330.  A launch takes 2^26 points at most, below the 2^32 threads it may have.
+    // 1300 / 1470 / 1330.  A launch takes 2^26 points at most, whose threads' indices fit 32 bits.
     constexpr long long kFew = 32768, kLaunch = 1 << 26;
     for (long long first = 0; first < npts; first += kLaunch) {
         const int m = (int)std::min<long long>(npts - first, kLaunch);

@@ -23,6 +23,8 @@
 // below the list's capacity: the host learns the totals after the evaluation
 // and runs it again with larger lists when one did not fit, so that no host
 // wait sits between the passes.
+#include <algorithm>
+
 #include "device_common.h"
 #include "kernels.h"
 
@@ -290,37 +292,39 @@ __global__ void __launch_bounds__(256) k_trimer_pass(int n, const int* __restric
                                                      const int2* __restrict__ lower, int full_list,
                                                      long long* __restrict__ count, const long long* __restrict__ offset,
                                                      int* __restrict__ trip, int lower_cap, long long cap) {
-    const int a = (blockIdx.x * blockDim.x + threadIdx.x) / kGT, lane = threadIdx.x % kGT;
-    if (a > lower_cap) return;  // uniform over the group
-    const int nl = lo_start[n];
-    // past the list's end, or an incomplete lower list (it overflowed its capacity):
-    // nothing to read; the evaluation is then run again with a larger one
-    if (a >= nl || nl > lower_cap) {
-        if (count && lane == 0) count[a] = 0;
-        return;
-    }
-    const int2 ij = lower[a];
-    const d3 pi = opos(pos, idx, ij.x), pj = opos(pos, idx, ij.y);
+    const int lane = threadIdx.x % kGT, nl = lo_start[n];
     const unsigned long long gb = group_bits<kGT>(), below = lanes_below();
-    long long c = 0;
-    const long long o = offset ? offset[a] : 0;
-    const int e = lo_start[ij.y + 1];
-    for (int b = lo_start[ij.y]; b < e; b += kGT) {
-        const bool act = b + lane < e;
-        const int k = act ? lower[b + lane].y : 0;
-        const bool ok = act && (full_list || trimer_active(pi, pj, opos(pos, idx, k), g));
-        const unsigned long long bits = __ballot(ok) & gb;
-        if (ok && trip) {
-            const long long t = o + c + __popcll(bits & below);
-            if (t < cap) {
-                trip[3 * t] = ij.x;
-                trip[3 * t + 1] = ij.y;
-                trip[3 * t + 2] = k;
-            }
+    const long long step = (long long)gridDim.x * blockDim.x / kGT;
+    for (long long a = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kGT; a <= lower_cap;
+         a += step) {  // uniform over the group
+        // past the list's end, or an incomplete lower list (it overflowed its capacity):
+        // nothing to read; the evaluation is then run again with a larger one
+        if (a >= nl || nl > lower_cap) {
+            if (count && lane == 0) count[a] = 0;
+            continue;
         }
-        c += __popcll(bits);
+        const int2 ij = lower[a];
+        const d3 pi = opos(pos, idx, ij.x), pj = opos(pos, idx, ij.y);
+        long long c = 0;
+        const long long o = offset ? offset[a] : 0;
+        const int e = lo_start[ij.y + 1];
+        for (int b = lo_start[ij.y]; b < e; b += kGT) {
+            const bool act = b + lane < e;
+            const int k = act ? lower[b + lane].y : 0;
+            const bool ok = act && (full_list || trimer_active(pi, pj, opos(pos, idx, k), g));
+            const unsigned long long bits = __ballot(ok) & gb;
+            if (ok && trip) {
+                const long long t = o + c + __popcll(bits & below);
+                if (t < cap) {
+                    trip[3 * t] = ij.x;
+                    trip[3 * t + 1] = ij.y;
+                    trip[3 * t + 2] = k;
+                }
+            }
+            c += __popcll(bits);
+        }
+        if (count && lane == 0) count[a] = c;
     }
-    if (count && lane == 0) count[a] = c;
 }
 
 // out[i] = off[start[i]], i <= n: offsets per molecule from those per lower pair
@@ -367,9 +371,12 @@ void launch_lower_pass(hipStream_t s, int n, const int* idx, const double* pos, 
 void launch_trimer_pass(hipStream_t s, int n, const int* idx, const double* pos, ListGeom g, const int* lo_start,
                         const int2* lower, int full_list, long long* count, const long long* offset, int* trip,
                         int lower_cap, long long cap) {
+    // at most 2^17 blocks, whose groups stride over longer lists (from 2^29 pairs on a thread's index would not fit
+    // the 32 bits of blockIdx.x * blockDim.x)
+    const int blocks = std::min(nblk((lower_cap + 1LL) * kGT, 256), 1 << 17);
     if (n > 0)
-        hipLaunchKernelGGL(k_trimer_pass, nblk((lower_cap + 1LL) * kGT, 256), 256, 0, s, n, idx, pos, g, lo_start, lower,
-                           full_list, count, offset, trip, lower_cap, cap);
+        hipLaunchKernelGGL(k_trimer_pass, blocks, 256, 0, s, n, idx, pos, g, lo_start, lower, full_list, count, offset,
+                           trip, lower_cap, cap);
 }
 void launch_offsets_of(hipStream_t s, int n, const int* start, int limit, const long long* off, long long* out) {
     if (n > 0) hipLaunchKernelGGL(k_offsets_of, nblk(n + 1, 256), 256, 0, s, n, start, limit, off, out);
