@@ -185,6 +185,7 @@ struct mbpol_context {
     mbpol::DevBuf trip_mol_off;                 // offsets per molecule (independent groups)
     long long trip_cap = 0;
     mbpol::DevBuf pip_shares, pip_points;  // PipScratch of the 2- and 3-body kernels
+    bool pip2_join = true, pip3_join = true;  // whether their joining kernels are launched (list_check)
     int lists_built = 0;        // lists built by this evaluation: 1 dimers, 2 trimers
     mbpol::DevBuf results_stage;  // energies and list lengths gathered for the one read-back (11 u64, every system)
 

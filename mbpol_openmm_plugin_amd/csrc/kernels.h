@@ -127,7 +127,10 @@ struct PipScratch {
     void* shares;
     double* points;
     int slots;  // compute units of the device
+    bool join;  // whether the joining kernel is launched (pip_splits of a list it was not launched for: run again)
 };
+// whether units of a list of n dimers or trimers are spread over several blocks
+inline bool pip_splits(long long n, int slots) { return 2 * ((n + 63) / 64) <= slots; }
 // the polynomials through their relabelling groups (pip_orbit_loop.h), FP32 and FP64
 MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f32, int2, const PipScratch& scratch, );
 MBPOL_PIP_LAUNCHER(launch_twobody_orbit_f64, int2, const PipScratch& scratch, );

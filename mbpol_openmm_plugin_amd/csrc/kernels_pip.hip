@@ -730,10 +730,9 @@ __global__ void __launch_bounds__(64) k_threebody(long long nt, const long long*
 // finer until the waves would meet on a SIMD again (8 waves in one block on one CU
 // gained nothing over 4).  One wave per unit through all passes (2-body: term by
 // term) took 207 us for 101 trimers, 238 for 13,641, 566 for 139,535; 93 for 91 dimers,
-// 93 for 4612, 105 for 42,250.  Both kernels here: 101 trimers 38-51 (beside
-// the other terms, or alone), 776 41, 9204 88, 134,272 638 in a grid of one wave a SIMD;
-// 91 dimers 40, 2016 44, 42,250 86 -- the join is 4-6 of each, and an idle launch for
-// long lists.
+// 93 for 4612, 105 for 42,250.  Here, with the join (4-5 us) where there is one: 101
+// trimers 38-48 (beside the other terms, or alone), 776 40, 9204 84-91, 134,272 633 in a
+// grid of one wave a SIMD; 91 dimers 37, 2016 42, 42,250 81.
 // ---------------------------------------------------------------------------
 #if PIP_BODY == 2
 constexpr int kPoints = 10, kVars = 31, kMols = 2, kPassAll = pip2b_npass;
@@ -973,15 +972,18 @@ static inline int join_grid(long long n, int slots) { return (int)std::min<long 
 #define PIP_LAUNCH(kern, n, s, np, ndev, list, idx, ...)                                                             \
     do {                                                                                                             \
         const int blocks = split_grid(n, max_blocks, scratch.slots), joins = join_grid(n, scratch.slots);            \
-        if (ev.start) { /* the span of both */                                                                       \
-            hipExtLaunchKernelGGL(k_pip_split, blocks, 64 * P, 0, s, ev.start, nullptr, 0, scratch, np, ndev, list,  \
-                                  idx, __VA_ARGS__);                                                                 \
+        const hipEvent_t split_stop = scratch.join ? nullptr : ev.stop; /* a timed span ends with the last kernel */ \
+        if (ev.start)                                                                                                \
+            hipExtLaunchKernelGGL(k_pip_split, blocks, 64 * P, 0, s, ev.start, split_stop, 0, scratch, np, ndev,     \
+                                  list, idx, __VA_ARGS__);                                                           \
+        else                                                                                                         \
+            hipLaunchKernelGGL(k_pip_split, blocks, 64 * P, 0, s, scratch, np, ndev, list, idx, __VA_ARGS__);        \
+        if (!scratch.join) break;                                                                                    \
+        if (ev.start)                                                                                                \
             hipExtLaunchKernelGGL(k_pip_join, joins, 64 * P, 0, s, nullptr, ev.stop, 0, scratch, np, ndev, list,     \
                                   idx, force, energy, eunit);                                                        \
-        } else {                                                                                                     \
-            hipLaunchKernelGGL(k_pip_split, blocks, 64 * P, 0, s, scratch, np, ndev, list, idx, __VA_ARGS__);        \
+        else                                                                                                         \
             hipLaunchKernelGGL(k_pip_join, joins, 64 * P, 0, s, scratch, np, ndev, list, idx, force, energy, eunit); \
-        }                                                                                                            \
     } while (0)
 #else
 #define PIP_SCRATCH

@@ -826,8 +826,16 @@ static int list_check(mbpol_context* ctx, bool& redo) {
     const mbpol_system& s = ctx->sys;
     const long long* hc = static_cast<const long long*>(ctx->h_counts);
     redo = false;
+    // The kernels that join the units spread over several blocks are left out while the lists are longer than
+    // twice what is spread: an idle launch costs 5 us of a call.  A list that has shrunk below that at once is
+    // evaluated again.
+    auto joins = [&](long long n, bool& join) {
+        if (n > 0 && pip_splits(n, ctx->cus) && !join) redo = true;
+        join = pip_splits(n / 2, ctx->cus);
+    };
     if (ctx->lists_built & 1) {
         const long long nd = hc[16];
+        if (ctx->pip2_kernel == 0) joins(nd, ctx->pip2_join);
         if (nd > ctx->dimer_cap) {
             HIP_TRY(ctx->dimers.ensure(sizeof(int2) * (nd + nd / 4 + 64)));
             ctx->dimer_cap = nd + nd / 4 + 64;
@@ -837,6 +845,7 @@ static int list_check(mbpol_context* ctx, bool& redo) {
     }
     if (ctx->lists_built & 2) {
         const long long nl = hc[17], nt = hc[18];
+        if (nl <= ctx->lower_cap && ctx->pip3_kernel == 0) joins(nt, ctx->pip3_join);
         if (nl > ctx->lower_cap) {
             HIP_TRY(ctx->lower.ensure(sizeof(int2) * (nl + nl / 4 + 64)));
             ctx->lower_cap = (int)(nl + nl / 4 + 64);
@@ -901,7 +910,8 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
     // terms cancel to ~1e-3 of their magnitudes, so FP32 evaluation loses three
     // digits of the 2- and 3-body energies.
     const bool dp = ctx->precision != MBPOL_PRECISION_SINGLE_PIP;
-    const PipScratch scratch{ctx->pip_shares.p, ctx->pip_points.as<double>(), ctx->cus};
+    const PipScratch scratch2{ctx->pip_shares.p, ctx->pip_points.as<double>(), ctx->cus, ctx->pip2_join};
+    const PipScratch scratch3{ctx->pip_shares.p, ctx->pip_points.as<double>(), ctx->cus, ctx->pip3_join};
     auto run2 = [&]() -> int {
         if (do2) {
             const int per = s.tb_method == MBPOL_CUTOFF_PERIODIC;
@@ -915,7 +925,7 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
                                                                eu2, ctx->pip_blocks);
             else
                 (dp ? launch_twobody_orbit_f64 : launch_twobody_orbit_f32)(sr, ctx->dimer_cap, nd, dl, ti, pos, per, box, F,
-                                                                           E + 1, scratch, ev, eu2, ctx->pip_blocks);
+                                                                           E + 1, scratch2, ev, eu2, ctx->pip_blocks);
             timer_kernel_done(ctx, T_TWOBODY, ev);
             // dimers are listed by their first molecule, so a group's dimers are consecutive
             if (G)
@@ -937,7 +947,7 @@ static int short_range(mbpol_context* ctx, hipStream_t sr, uint32_t comp) {
                 launch_threebody_f64(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2, ev, eu3, cap);
             else
                 (dp ? launch_threebody_orbit_f64 : launch_threebody_orbit_f32)(sr, nt, ntd, tr, ti, pos, per, box, F, E + 2,
-                                                                               scratch, ev, eu3, cap);
+                                                                               scratch3, ev, eu3, cap);
             timer_kernel_done(ctx, T_THREEBODY, ev);
             if (G) {
                 const int n3 = (int)s.th_idx.size() / 3;
@@ -1217,6 +1227,7 @@ static void graph_key(const mbpol_context* ctx, double* forces_dev_out, uint32_t
     key[6] = ctx->trip_cap;
     key[7] = ctx->graph_steps;
     key[8] = (long long)(intptr_t)ctx->pos.p;
+    key[13] = 2 * ctx->pip3_join + ctx->pip2_join;
     if ((comp & MBPOL_ELECTROSTATICS) && ctx->elec) elec_graph_key(ctx, key + 9);
 }
 

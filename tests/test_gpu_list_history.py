@@ -77,3 +77,25 @@ def test_lengths_cover_every_split(mb, monkeypatch):
         print(keep, units2, units3, flush=True)
     assert three == {1, 2, 3, 6}
     assert 2 in two
+
+
+@pytest.mark.parametrize('graph', [False, True])
+def test_short_list_after_long_ones(mb, monkeypatch, graph):
+    """The kernel that joins units of several blocks is left out of long lists' launches: a list that turns
+    short at once, eagerly or in a replayed graph, still gives a fresh Context's bits, and so do long ones."""
+    box = mb.systems.config2()[0][:1500]
+    few, some = sparse_box(box, 40), sparse_box(box, 400)
+    want = {}
+    for k, w in (('few', few), ('some', some), ('all', box)):
+        want[k] = evaluate(mb, context(mb, len(box), 6, 'orbit', monkeypatch), w, 6)
+    assert 64 * 128 < want['all'][2]['num_dimers'] and want['few'][2]['num_dimers'] <= 64 * 128
+    ctx = context(mb, len(box), 6, 'orbit', monkeypatch)
+    ctx.setGraph(graph)
+    waters = {'few': few, 'some': some, 'all': box}
+    for k in ('all', 'all', 'all', 'few', 'few', 'all', 'all', 'some', 'few', 'some', 'all', 'all', 'all', 'few'):
+        e, f, st = evaluate(mb, ctx, waters[k], 6)
+        print(k, st['num_dimers'], st['num_trimers'], e, flush=True)
+        assert e == want[k][0]
+        assert np.array_equal(f, want[k][1])
+    if graph:
+        assert ctx.getTuning('graph_replays') > 0
