@@ -68,8 +68,8 @@ void launch_site_lists(hipStream_t s, int n, const double* pos, const double* po
 void launch_prefactors_field(hipStream_t s, int npol, const int* polidx, const double* pos, SiteParams S, ElecParams P,
                              const ElecRows& R, double2* pf, double* field);
 void launch_site_spline_table(hipStream_t s, int n, const double* pos, ElecParams P, int* g0tab, double* sptab);
-// spreading table by grid line, each in nseg segments (2 grid.x grid.y nseg rows): stage 0 counts the rows' entries, stage 1 (after a scan
-// of the counts into rowstart) fills them; rowcount and rowfill start at zero
+// spreading table by grid line, each in nseg segments (2 grid.x grid.y nseg rows): stage 0 counts the rows'
+// entries, stage 1 (after a scan of the counts into rowstart) fills them; rowcount and rowfill start at zero
 void launch_line_table(hipStream_t s, int stage, int n, const int* g0tab, const double* sptab, const double* pol,
                        const double* q, ElecParams P, int nseg, int* rowcount, const int* rowstart, int* rowfill, int* code,
                        int2* sz, double* coef);

@@ -664,8 +664,8 @@ __global__ void k_site_spline_table(int n, const double* __restrict__ pos, ElecP
 // and the z splines v0, v1 of the site.  The table lists, line by line and in a line
 // segment by segment of its points (nseg, by the first z), the sites (in index order:
 // every sum has a fixed order) with their first z and c: the lines' rows first for the
-// polarisable sites, then for the other charged ones.  A seventh of the memory of a table by grid point (32 bytes for 5 points
-// against 28 for each), and of the work to build it.
+// polarisable sites, then for the other charged ones.  A seventh of the memory of a table
+// by grid point (32 bytes for 5 points against 28 for each), and of the work to build it.
 // ---------------------------------------------------------------------------
 // row of entry c (0..24) of site i; -1 when the site adds nothing
 __device__ __forceinline__ int line_row(int i, int c, const int* __restrict__ g0tab, const double* __restrict__ pol,
